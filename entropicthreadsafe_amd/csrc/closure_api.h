@@ -128,6 +128,22 @@ int run_grad(tslb_closure *m, int nb, int64_t ntot, float t_scale) {
   return TSLB_OK;
 }
 
+// inputs of every node of a grid; phi (field fphi) in two-component runs only
+template <typename View>
+void launch_features(const View &v, const Params &p, int fu, int fphi, float *feat, long long fstride, long long foff,
+                     int ncu, hipStream_t st) {
+  // z-chunks of 32 planes, shorter while there are fewer than four blocks per
+  // CU (each chunk loads two planes more than it has)
+  const long long tiles = (long long)((p.nx + FTX - 1) / FTX) * ((p.ny + FTY - 1) / FTY);
+  int zc = 32;
+  while (zc > 2 && tiles * ((p.nz + zc - 1) / zc) < 4LL * ncu) zc /= 2;
+  const dim3 g((unsigned)(tiles * ((p.nz + zc - 1) / zc)));
+  if (p.ncomp == 2)
+    hipLaunchKernelGGL((k_features<View, true>), g, dim3(FNT), 0, st, v, p, fu, fphi, feat, fstride, foff, zc);
+  else
+    hipLaunchKernelGGL((k_features<View, false>), g, dim3(FNT), 0, st, v, p, fu, fphi, feat, fstride, foff, zc);
+}
+
 // closure fields of every node of c from its current state (before a collision)
 int launch_closure(tslb_ctx *c) {
   tslb_closure *m = c->model;
@@ -135,9 +151,8 @@ int launch_closure(tslb_ctx *c) {
   const long long n = (long long)c->n;
   with_storage(c, [&](auto tag) {
     using S = decltype(tag);
-    StateView<S> v{(const S *)c->buf[c->cur], (long long)c->fs};
-    hipLaunchKernelGGL(k_features<StateView<S>>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, c->stream, v,
-                       p, (int)TSLB_U, p.ncomp == 2 ? (int)TSLB_PHI : -1, c->cfeat, n, 0LL);
+    StateView<S> v{(const S *)c->buf[c->cur]};
+    launch_features(v, p, TSLB_U, TSLB_PHI, c->cfeat, n, 0, c->ncu, c->stream);
     return 0;
   });
   hipLaunchKernelGGL(k_mlp_infer, dim3(grid_for_tiles((n + 15) / 16)), dim3(256), 0, c->stream, c->cfeat, n, n,
@@ -255,14 +270,13 @@ int tslb_closure_add_samples(tslb_closure *m, tslb_ctx *c, int factor) {
   const unsigned g = (unsigned)((nc + 255) / 256);
   with_storage(c, [&](auto tag) {
     using S = decltype(tag);
-    StateView<S> v{(const S *)c->buf[c->cur], (long long)c->fs};
+    StateView<S> v{(const S *)c->buf[c->cur]};
     hipLaunchKernelGGL(k_box_filter<S>, dim3(g), dim3(256), 0, c->stream, v, c->kp, r, m->coarse, (long long)nc,
                        m->aux, (long long)m->cap, (long long)m->ns);
     return 0;
   });
   PlainView cv{m->coarse, (long long)nc};
-  hipLaunchKernelGGL(k_features<PlainView>, dim3(g), dim3(256), 0, c->stream, cv, pc, 1, c->prm.ncomp == 2 ? 4 : -1,
-                     m->feat, (long long)m->cap, (long long)m->ns);
+  launch_features(cv, pc, 1, 4, m->feat, (long long)m->cap, (long long)m->ns, c->ncu, c->stream);
   HIPCK(hipGetLastError());
   HIPCK(hipStreamSynchronize(c->stream));
   m->ns += nc;

@@ -474,19 +474,33 @@ __global__ __launch_bounds__(256) void k_mlp_adam(float *__restrict__ th, const 
 }
 
 // Field views for the filter and input kernels: the lattice state (storage
-// type S, per-field scale) or a plain FP32 SoA buffer.
+// type S, per-field scale) or a plain FP32 SoA buffer.  `col` locates a column
+// (x, y), `get` reads field q of its node in plane z.
 template <typename S>
 struct StateView {
   const S *base;
-  long long fs;
-  __device__ __forceinline__ float get(int q, long long id, const Params &p) const {
-    return dec(base[q * fs + id], p, sgrp(q));
+  struct Col {
+    uint64_t off;  // in the moment layout
+    uint32_t xy;   // in the plain phi field
+  };
+  __device__ __forceinline__ Col col(int x, int y, const Params &p) const {
+    return Col{node_off<(int)sizeof(S)>(p, x, y), (uint32_t)(x + p.nx * y)};
+  }
+  __device__ __forceinline__ float get(int q, const Col &c, int z, const Params &p) const {
+    if (q == TSLB_PHI) return ldv(base, (uint64_t)p.phi0 + (uint64_t)((long long)p.nx * p.ny * z) + c.xy, p, q);
+    return ldv(base, plane_off(p, z) + c.off + (uint32_t)(q * kRowNodes), p, q);
   }
 };
 struct PlainView {
   const float *base;
   long long fs;
-  __device__ __forceinline__ float get(int q, long long id, const Params &) const { return base[q * fs + id]; }
+  struct Col {
+    uint32_t xy;
+  };
+  __device__ __forceinline__ Col col(int x, int y, const Params &p) const { return Col{(uint32_t)(x + p.nx * y)}; }
+  __device__ __forceinline__ float get(int q, const Col &c, int z, const Params &p) const {
+    return base[q * fs + (long long)p.nx * p.ny * z + c.xy];
+  }
 };
 
 // Box filter of a fine lattice by r^3 blocks: coarse rho_bar - 1, Favre
@@ -501,18 +515,18 @@ __global__ __launch_bounds__(256) void k_box_filter(StateView<S> f, Params p, in
   if (t >= nc) return;
   const int I = (int)(t % ncx), J = (int)((t / ncx) % ncy), K = (int)(t / ((long long)ncx * ncy));
   (void)ncz;
-  const long long plane = (long long)p.nx * p.ny;
   double sr = 0, su = 0, sv = 0, sw = 0, sp = 0;
   for (int k = 0; k < r; k++)
     for (int j = 0; j < r; j++)
       for (int i = 0; i < r; i++) {
-        const long long id = (long long)(I * r + i) + (long long)p.nx * (J * r + j) + plane * (K * r + k);
-        const float rho = 1.f + f.get(TSLB_RHO, id, p);
+        const auto c = f.col(I * r + i, J * r + j, p);
+        const int z = K * r + k;
+        const float rho = 1.f + f.get(TSLB_RHO, c, z, p);
         sr += rho;
-        su += (double)rho * f.get(TSLB_U, id, p);
-        sv += (double)rho * f.get(TSLB_V, id, p);
-        sw += (double)rho * f.get(TSLB_W, id, p);
-        if (p.ncomp == 2) sp += f.get(TSLB_PHI, id, p);
+        su += (double)rho * f.get(TSLB_U, c, z, p);
+        sv += (double)rho * f.get(TSLB_V, c, z, p);
+        sw += (double)rho * f.get(TSLB_W, c, z, p);
+        if (p.ncomp == 2) sp += f.get(TSLB_PHI, c, z, p);
       }
   const double inv = 1.0 / ((double)r * r * r);
   const double rb = sr * inv, ut = su / sr, vt = sv / sr, wt = sw / sr;
@@ -520,10 +534,11 @@ __global__ __launch_bounds__(256) void k_box_filter(StateView<S> f, Params p, in
   for (int k = 0; k < r; k++)
     for (int j = 0; j < r; j++)
       for (int i = 0; i < r; i++) {
-        const long long id = (long long)(I * r + i) + (long long)p.nx * (J * r + j) + plane * (K * r + k);
-        const double rho = 1.0 + f.get(TSLB_RHO, id, p);
-        const double du = f.get(TSLB_U, id, p) - ut, dv = f.get(TSLB_V, id, p) - vt,
-                     dw = f.get(TSLB_W, id, p) - wt;
+        const auto c = f.col(I * r + i, J * r + j, p);
+        const int z = K * r + k;
+        const double rho = 1.0 + f.get(TSLB_RHO, c, z, p);
+        const double du = f.get(TSLB_U, c, z, p) - ut, dv = f.get(TSLB_V, c, z, p) - vt,
+                     dw = f.get(TSLB_W, c, z, p) - wt;
         txx += rho * du * du;
         tyy += rho * dv * dv;
         tzz += rho * dw * dw;
@@ -550,44 +565,90 @@ __global__ __launch_bounds__(256) void k_box_filter(StateView<S> f, Params p, in
 // S from the isotropic gradient (3 sum_l w_l c_l f(x + c_l), the stencil of
 // grad_axis) of (u, v, w), grad(phi), phi; the nearest
 // interior node across a wall.  Velocity at fields fu..fu+2 and phi at field
-// fphi of a SoA source (phi absent: fphi < 0).  Output SoA 10 x fstride at
+// fphi of a source (without PHI: phi = 0).  Output SoA 10 x fstride at
 // column offset foff.
-template <typename Src>
-__global__ __launch_bounds__(256) void k_features(Src f, Params p, int fu, int fphi, float *__restrict__ feat,
-                                                  long long fstride, long long foff) {
-  const long long n = (long long)p.nx * p.ny * p.nz;
-  const long long t = (long long)blockIdx.x * 256 + threadIdx.x;
-  if (t >= n) return;
-  const int i = (int)(t % p.nx), j = (int)((t / p.nx) % p.ny), k = (int)(t / ((long long)p.nx * p.ny));
-  // 3 sum_l w_l c_l f(x + c_l) for u, v, w and phi, one neighbour at a time
-  float gu[3] = {0.f, 0.f, 0.f}, gv[3] = {0.f, 0.f, 0.f}, gw[3] = {0.f, 0.f, 0.f}, gp[3] = {0.f, 0.f, 0.f};
-#pragma unroll 1
-  for (int l = 1; l < 27; l++) {
-    const int cx = kCX[l], cy = kCY[l], cz = kCZ[l];
-    const long long id = (long long)clampw(i + cx, p.nx, p.px) +
-                         (long long)p.nx * (clampw(j + cy, p.ny, p.py) + (long long)p.ny * clampw(k + cz, p.nz, p.pz));
-    const float w3 = 3.f * wgt(l);
-    const float c[3] = {w3 * (float)cx, w3 * (float)cy, w3 * (float)cz};
-    const float u = f.get(fu, id, p), v = f.get(fu + 1, id, p), w = f.get(fu + 2, id, p);
-    const float ph = fphi >= 0 ? f.get(fphi, id, p) : 0.f;
+//
+// A 64x4 block marches a z-chunk.  It keeps four planes of its 66x6 footprint
+// in an LDS ring (25 KiB; the plane two ahead loads into registers meanwhile)
+// and forms the 12 sums of a node from 104 LDS reads, in the order of the
+// directions.  One thread per node reading its 26 neighbours from memory
+// took 79 us at 128^3 for its addresses and L1 reads; this one takes 34 us (84 MB
+// written and 34 MB read: 24 us at the rate of a copy).
+constexpr int FTX = 64, FTY = 4, FSW = FTX + 2, FSH = FTY + 2, FNSLOT = FSW * FSH, FNT = FTX * FTY;
+static_assert(FNSLOT <= 2 * FNT, "at most two footprint slots per thread");
+template <typename Src, bool PHI>
+__global__ __launch_bounds__(FNT) void k_features(Src f, Params p, int fu, int fphi, float *__restrict__ feat,
+                                                  long long fstride, long long foff, int zc) {
+  constexpr int NQ = PHI ? 4 : 3;
+  __shared__ float ring[4][NQ][FNSLOT];
+  const int tid = threadIdx.x, tx = tid % FTX, ty = tid / FTX;
+  const int tilx = (p.nx + FTX - 1) / FTX, tily = (p.ny + FTY - 1) / FTY;
+  int b = xcd_tile(blockIdx.x, gridDim.x);
+  const int x0 = b % tilx * FTX;
+  b /= tilx;
+  const int y0 = b % tily * FTY, z0 = b / tily * zc, z1 = min(z0 + zc, p.nz);
+  const int x = x0 + tx, y = y0 + ty;
+  const bool active = x < p.nx && y < p.ny, two = tid + FNT < FNSLOT;
+  auto column = [&](int sl) {
+    return f.col(clampw(x0 + sl % FSW - 1, p.nx, p.px), clampw(y0 + sl / FSW - 1, p.ny, p.py), p);
+  };
+  const auto c0 = column(tid), c1 = column(two ? tid + FNT : tid);
+  float n0[NQ], n1[NQ];
+  auto issue = [&](int z) {
+    const int gz = clampw(z, p.nz, p.pz);
 #pragma unroll
-    for (int a = 0; a < 3; a++) {
-      gu[a] = fmaf(c[a], u, gu[a]);
-      gv[a] = fmaf(c[a], v, gv[a]);
-      gw[a] = fmaf(c[a], w, gw[a]);
-      gp[a] = fmaf(c[a], ph, gp[a]);
+    for (int q = 0; q < NQ; q++) {
+      const int fq = q < 3 ? fu + q : fphi;
+      n0[q] = f.get(fq, c0, gz, p);
+      if (two) n1[q] = f.get(fq, c1, gz, p);
     }
+  };
+  auto commit = [&](int z) {
+    float(*d)[FNSLOT] = ring[(z - z0 + 4) & 3];
+#pragma unroll
+    for (int q = 0; q < NQ; q++) {
+      d[q][tid] = n0[q];
+      if (two) d[q][tid + FNT] = n1[q];
+    }
+  };
+  issue(z0 - 1);
+  commit(z0 - 1);
+  issue(z0);
+  commit(z0);
+  issue(z0 + 1);
+  // the slot of plane z + 1 held plane z - 3, last read before the previous
+  // barrier
+  for (int z = z0; z < z1; z++) {
+    commit(z + 1);
+    if (z + 2 <= z1) issue(z + 2);
+    __syncthreads();
+    if (!active) continue;
+    const int own = (ty + 1) * FSW + tx + 1;
+    float g[NQ][3];
+#pragma unroll
+    for (int q = 0; q < NQ; q++) g[q][0] = g[q][1] = g[q][2] = 0.f;
+#pragma unroll
+    for (int l = 1; l < 27; l++) {
+      const float *s = ring[(z + kCZ[l] - z0 + 4) & 3][0] + own + kCY[l] * FSW + kCX[l];
+      const float w3 = 3.f * wgt(l);
+#pragma unroll
+      for (int q = 0; q < NQ; q++) {
+        const float v = s[q * FNSLOT];
+        if (kCX[l]) g[q][0] = fmaf(w3 * (float)kCX[l], v, g[q][0]);
+        if (kCY[l]) g[q][1] = fmaf(w3 * (float)kCY[l], v, g[q][1]);
+        if (kCZ[l]) g[q][2] = fmaf(w3 * (float)kCZ[l], v, g[q][2]);
+      }
+    }
+    float *o = feat + foff + ((long long)p.nx * p.ny * z + (x + p.nx * y));
+    o[0] = g[0][0];
+    o[fstride] = g[1][1];
+    o[2 * fstride] = g[2][2];
+    o[3 * fstride] = 0.5f * (g[0][1] + g[1][0]);
+    o[4 * fstride] = 0.5f * (g[0][2] + g[2][0]);
+    o[5 * fstride] = 0.5f * (g[1][2] + g[2][1]);
+    o[6 * fstride] = PHI ? g[NQ - 1][0] : 0.f;
+    o[7 * fstride] = PHI ? g[NQ - 1][1] : 0.f;
+    o[8 * fstride] = PHI ? g[NQ - 1][2] : 0.f;
+    o[9 * fstride] = PHI ? ring[(z - z0 + 4) & 3][NQ - 1][own] : 0.f;
   }
-  const float ph = fphi >= 0 ? f.get(fphi, t, p) : 0.f;
-  const long long o = foff + t;
-  feat[o] = gu[0];
-  feat[fstride + o] = gv[1];
-  feat[2 * fstride + o] = gw[2];
-  feat[3 * fstride + o] = 0.5f * (gu[1] + gv[0]);
-  feat[4 * fstride + o] = 0.5f * (gu[2] + gw[0]);
-  feat[5 * fstride + o] = 0.5f * (gv[2] + gw[1]);
-  feat[6 * fstride + o] = gp[0];
-  feat[7 * fstride + o] = gp[1];
-  feat[8 * fstride + o] = gp[2];
-  feat[9 * fstride + o] = ph;
 }

@@ -132,7 +132,13 @@ struct Params {
   float sigma, sharp_c;
   float fx, fy, fz, lin_a;
   int z_chunk, tiles_x, tiles_y, nzc;
-  long long fs;             // element stride between the fields of a state buffer
+  long long fs;             // element stride of the plain per-node arrays (normals, curvature, closure)
+  // moment layout (node_off, plane_off), in stored values
+  int tiled;                // 1: tiles in superpages, 0: rows of 64 consecutive nodes
+  int zsh;                  // 2^zsh planes share a row of 64 nodes (lattices of at most 32 columns)
+  long long ps;             // stride of 2^zsh planes
+  long long phi0;           // offset of the plain phi field
+  int wide;                 // 1: k_fused<..., WIDE> (planes beyond 32-bit byte offsets, zsh > 0)
   int gwall;                // 1: walls absorb phase populations (jet boundary)
   float inua, inub;         // colour model: 1/nu of components A and B
   float beta;               // colour model: recolouring parameter
@@ -281,30 +287,90 @@ __device__ __forceinline__ float dec(S x, const Params &p, int g) {
   else return to_f(x) * p.isc[g];
 }
 
-template <typename S>
-struct FieldsT {
-  S *f[TSLB_NFIELDS];
+// ---------------------------------------------------------------------------
+// Layout of a state buffer.  The ten hydrodynamic fields are interleaved in
+// rows of 64 nodes: row = [field q][node i], 64 values each, so that the ten
+// loads of a source lie at constant offsets from one address.  phi (psi) is a
+// plain field behind them (its readers take phi alone).
+//
+// The fused pass is bound by HBM in FP32 storage, and what limits it there is
+// DRAM page locality: the blocks of a launch drift apart, so a page that holds
+// pieces for several blocks is opened once for each.  A contiguous 256 KiB
+// spreads over all channels, 2 KiB of a DRAM page per channel at a stride of
+// 32 KiB (found by timing: copying 20 KiB records in random order moves 5.1
+// TB/s when a record is contiguous and 6.1 TB/s when its eight rows lie 32 KiB
+// apart; 16 and 64 KiB are close, 8 and 128 KiB lose it).  So the eight rows of
+// a 64x8 tile-plane sit 32 KiB apart (`kPitch`) and a block opens its own pages
+// only; 12 tiles (25 in 16-bit storage) share the eight 32 KiB lines of such a
+// superpage.  The access pattern of the fused pass alone (loads with halo, nt
+// stores, no arithmetic) takes, plain fields / rows in sequence / superpages:
+// 512x256x256 FP32 0.583 / 0.524 / 0.491 ms, 512^3 2.20 / 2.10 / 1.96 ms,
+// 512^3 FP16 1.40 / 1.33 / 1.16 ms.
+//
+// Lattices whose tiles would be padded to more than half as much again (narrow
+// or shallow ones) take the rows in sequence over the nodes of a plane
+// instead (`tiled` = 0), several planes to a row where a plane has at most 32
+// nodes, so that no shape needs much more memory than its nodes.
+// ---------------------------------------------------------------------------
+constexpr int NIL = 10;                       // interleaved fields
+constexpr int kRowNodes = 64;                 // nodes of a row
+constexpr int kRowLen = NIL * kRowNodes;      // values of a row
+constexpr int kLineBytes = 32768;             // distance of the rows of a tile in a superpage
+__host__ __device__ constexpr int line_len(int es) { return kLineBytes / es; }
+__host__ __device__ constexpr int line_tiles(int es) { return kLineBytes / (kRowLen * es); }
+// offset of node (x, y) in its plane and of plane z in the buffer, field 0;
+// field q < 10 sits q * kRowNodes values further
+template <int ES>
+__host__ __device__ inline uint64_t node_off(const Params &p, int x, int y) {
+  if (p.tiled) {
+    const uint32_t t = (uint32_t)(y / TY) * (uint32_t)p.tiles_x + (uint32_t)(x / TX);
+    const uint32_t sp = t / (uint32_t)line_tiles(ES), r = t - sp * (uint32_t)line_tiles(ES);
+    return (uint64_t)(sp * (uint32_t)TY + (uint32_t)(y % TY)) * line_len(ES) + r * kRowLen + x % TX;
+  }
+  const uint32_t xy = (uint32_t)(x + p.nx * y);
+  return (uint64_t)(xy / kRowNodes) * kRowLen + xy % kRowNodes;
+}
+__host__ __device__ inline uint64_t plane_off(const Params &p, int z) {
+  return (uint64_t)(z >> p.zsh) * (uint64_t)p.ps + (uint32_t)((z & ((1 << p.zsh) - 1)) * p.nx * p.ny);
+}
+// offset of field q of node (x, y, z)
+template <int ES>
+__host__ __device__ inline uint64_t mom_off(const Params &p, int q, int x, int y, int z) {
+  if (q == TSLB_PHI) return (uint64_t)p.phi0 + (uint64_t)((long long)p.nx * p.ny * z + (x + p.nx * y));
+  return plane_off(p, z) + node_off<ES>(p, x, y) + (uint32_t)(q * kRowNodes);
+}
+struct Node {
+  int x, y, z;
 };
-template <typename S>
-struct CFieldsT {
-  const S *f[TSLB_NFIELDS];
-};
+__device__ __forceinline__ Node node_of(const Params &p, int id) {
+  const int row = id / p.nx;
+  return Node{id - row * p.nx, row % p.ny, row / p.ny};
+}
 
-// scaled field access
+// scaled access to a stored value
 template <typename S>
-__device__ __forceinline__ float ldf(const S *__restrict__ a, int id, const Params &p, int q) {
-  return dec(a[id], p, sgrp(q));
+__device__ __forceinline__ float ldv(const S *__restrict__ a, uint64_t o, const Params &p, int q) {
+  return dec(a[o], p, sgrp(q));
 }
 template <typename S>
-__device__ __forceinline__ void stf(S *__restrict__ a, int id, float v, const Params &p, int q) {
+__device__ __forceinline__ void stv(S *__restrict__ a, uint64_t o, float v, const Params &p, int q) {
   if constexpr (sizeof(S) == 4) {
-    a[id] = from_f<S>(v);
+    a[o] = from_f<S>(v);
   } else {
     if constexpr (std::is_same<S, fx16_t>::value) {
       if (!(fabsf(v * p.sc[sgrp(q)]) <= 32767.5f) && p.sat) atomicAdd(p.sat, 1u);
     }
-    a[id] = from_f<S>(v * p.sc[sgrp(q)]);
+    a[o] = from_f<S>(v * p.sc[sgrp(q)]);
   }
+}
+// and to a moment of a state buffer
+template <typename S>
+__device__ __forceinline__ float ldf(const S *__restrict__ st, int q, int x, int y, int z, const Params &p) {
+  return ldv(st, mom_off<(int)sizeof(S)>(p, q, x, y, z), p, q);
+}
+template <typename S>
+__device__ __forceinline__ void stf(S *__restrict__ st, int q, int x, int y, int z, float v, const Params &p) {
+  stv(st, mom_off<(int)sizeof(S)>(p, q, x, y, z), v, p, q);
 }
 
 __device__ __forceinline__ int wrapc(int g, int n) {
@@ -390,7 +456,19 @@ struct ArraySink {
 // f(+1) = m2 + m1 costs three operations per triple.
 // The raw moments M[a][b][c] (scaled as above) of one source from its
 // moments (rho - 1, u, Pi), the equilibrium velocity V and the additive force.
-template <bool ADD>
+// The off-diagonal a2 = rho Va Vb + (1-omega) Pab are sums of two products, of
+// which one can be fused.  Left to the compiler, which one varied with the
+// code around it; so it is written out, as each kernel has had it.
+enum A2Form {
+  A2_VV,   // rho Va Vb fused
+  A2_PXY,  // xy: (1-omega) Pxy fused; xz, yz: rho Va Vb fused
+  A2_SUM   // neither
+};
+__device__ __forceinline__ float sum_of_rounded(float a, float b) {
+#pragma clang fp contract(off)
+  return a + b;
+}
+template <bool ADD, A2Form A2>
 __device__ __forceinline__ void raw_moments(float drho, float ux, float uy, float uz, float Pxx, float Pyy,
                                             float Pzz, float Pxy, float Pxz, float Pyz, float Vx, float Vy,
                                             float Vz, float fx, float fy, float fz, float om1,
@@ -407,7 +485,10 @@ __device__ __forceinline__ void raw_moments(float drho, float ux, float uy, floa
   }
   const float rVxy = rVx * Vy, rVxz = rVx * Vz, rVyz = rVy * Vz;
   const float a2xx = fmaf(rVx, Vx, Bxx), a2yy = fmaf(rVy, Vy, Byy), a2zz = fmaf(rVz, Vz, Bzz);
-  const float a2xy = rVxy + Bxy, a2xz = rVxz + Bxz, a2yz = rVyz + Byz;
+  const float a2xy = A2 == A2_PXY ? fmaf(om1, Pxy, rVxy)
+                                  : (A2 == A2_VV ? fmaf(rVx, Vy, Bxy) : sum_of_rounded(rVxy, Bxy));
+  const float a2xz = A2 == A2_SUM ? sum_of_rounded(rVxz, Bxz) : fmaf(rVx, Vz, Bxz);
+  const float a2yz = A2 == A2_SUM ? sum_of_rounded(rVyz, Byz) : fmaf(rVy, Vz, Byz);
   // rho Va Va Vb taken as (rho Va Vb) Va
   const float a3xxy = fmaf(rVxy, Vx, fmaf(uy, Bxx, 2.f * ux * Bxy));
   const float a3xxz = fmaf(rVxz, Vx, fmaf(uz, Bxx, 2.f * ux * Bxz));
@@ -453,11 +534,11 @@ __device__ __forceinline__ void raw_moments(float drho, float ux, float uy, floa
   M[2][2][2] = fmaf(0.25f * c9, s200_020 + M[0][0][2], drho * (-1.f / 108.f));
 }
 
-template <bool ADD, typename Sink>
+template <bool ADD, A2Form A2, typename Sink>
 __device__ __forceinline__ void all_pops_mt(const float *m, float Vx, float Vy, float Vz,
                                             const Params &p, Sink &h, float om1) {
   float M[3][3][3];
-  raw_moments<ADD>(m[0], m[1], m[2], m[3], m[4], m[5], m[6], m[7], m[8], m[9], Vx, Vy, Vz, p.fx, p.fy, p.fz,
+  raw_moments<ADD, A2>(m[0], m[1], m[2], m[3], m[4], m[5], m[6], m[7], m[8], m[9], Vx, Vy, Vz, p.fx, p.fy, p.fz,
                    om1, M);
   // pass z: G[a][b][cz]
   float G[3][3][3];
@@ -512,7 +593,7 @@ __device__ __forceinline__ void all_pops_mt(const float *m, float Vx, float Vy, 
 struct NoAdj {
   __device__ __forceinline__ float operator()(int, int, float v) const { return v; }
 };
-template <bool ADD, typename Adj = NoAdj>
+template <bool ADD, A2Form A2, typename Adj = NoAdj>
 __device__ __forceinline__ void ring_pops(const float *m, float Vx, float Vy, float Vz, const Params &p,
                                           float om1, bool col, float sgn, float *const (&rq)[3],
                                           const Adj &adj = Adj{}) {
@@ -526,7 +607,7 @@ __device__ __forceinline__ void ring_pops(const float *m, float Vx, float Vy, fl
     fp = col ? p.fx : p.fy;
   }
   float M[3][3][3];
-  raw_moments<ADD>(m[0], uq, up, m[3], Pqq, Ppp, m[6], m[7], Pqz, Ppz, Vq, Vp, Vz, fq, fp, p.fz, om1, M);
+  raw_moments<ADD, A2>(m[0], uq, up, m[3], Pqq, Ppp, m[6], m[7], Pqz, Ppz, Vq, Vp, Vz, fq, fp, p.fz, om1, M);
   float K[3][3];
 #pragma unroll
   for (int a = 0; a < 3; a++)
@@ -769,45 +850,74 @@ __device__ __forceinline__ void st_off(T *__restrict__ base, uint32_t byte_off, 
   *(T *)((char *)base + byte_off) = v;
 }
 
-// One source plane gz: byte bases of the plane in the state buffer (field 0)
-// and in the normals buffer (n0); field q sits q field strides further.
+// One source plane gz of the plain arrays: byte bases in the normals buffer
+// (n0) and the closure fields; field q sits q field strides further.
 struct PlaneSrc {
-  const char *f;      // state plane, field 0
   const char *n;      // normals plane, n0
   const char *c;      // closure plane, nu_t
-  uint32_t pbS, pb4;  // plane bytes (storage type, float)
-  long long fsS, fs4; // field stride in bytes (storage type, float)
+  uint32_t pb4;       // plane bytes
+  long long fs4;      // field stride in bytes
 };
 
-// Loads of one source node.  offS / off4 are in-plane byte offsets; off4 is
-// kOOB where the tile-plane has no interface (the buffer then returns 0
-// without a memory access).
+// The ten moments of one node of a plane in the moment layout.  One buffer
+// descriptor covers the plane and the fields lie at constant distances from
+// the node's 32-bit byte offset, so a load is one instruction without address
+// arithmetic.  WIDE: planes beyond 32-bit byte offsets (4 GiB: 107 million
+// nodes in FP32) and planes that share rows take the general address in 64
+// bits; for all lattices that cost the two-component kernels 5 spilled
+// registers (512^3 emulsion 2.52 against 2.44 ms in FP32, 2.53 against 2.37 in
+// FP16).
 constexpr uint32_t kOOB = 0x80000000u;
-// The ten hydrodynamic moments of a source are loaded; phi (psi) of the two
-// component models comes from the fused pass's LDS ring instead.
+constexpr uint32_t kAnyByte = 0xffffffffu;  // no bound: every offset is of a node of the lattice
+template <bool WIDE>
+using lane_off_t = typename std::conditional<WIDE, uint64_t, uint32_t>::type;
+template <typename S, bool WIDE>
+__device__ __forceinline__ lane_off_t<WIDE> lane_off(const Params &p, int x, int y) {
+  const uint64_t o = node_off<(int)sizeof(S)>(p, x, y) * sizeof(S);
+  return (lane_off_t<WIDE>)o;
+}
+// keeps off + constant next to its use, where it folds into the instruction's
+// offset (as loop invariants the ten sums took ten registers and spilled)
+__device__ __forceinline__ void keep_here(uint32_t &off) { asm volatile("" : "+v"(off)); }
+template <typename S, bool WIDE>
+__device__ __forceinline__ void load_node(const S *st, const Params &p, int z, lane_off_t<WIDE> off, S (&v)[NIL]) {
+  if constexpr (WIDE) {
+    const S *pl = st + plane_off(p, z);
+#pragma unroll
+    for (int q = 0; q < NIL; q++) v[q] = *(const S *)((const char *)pl + off + q * kRowNodes * sizeof(S));
+  } else {
+    const rsrc_t r = rsrc(st + (uint64_t)(uint32_t)z * (uint32_t)p.ps, kAnyByte);
+    keep_here(off);
+#pragma unroll
+    for (int q = 0; q < NIL; q++) v[q] = bld<S>(r, off + q * kRowNodes * (uint32_t)sizeof(S));
+  }
+}
+// stores f(0) .. f(9), non-temporally
+template <typename S, bool WIDE, typename F>
+__device__ __forceinline__ void store_node(S *st, const Params &p, int z, lane_off_t<WIDE> off, const F &f) {
+  if constexpr (WIDE) {
+    S *pl = st + plane_off(p, z);
+#pragma unroll
+    for (int q = 0; q < NIL; q++) *(S *)((char *)pl + off + q * kRowNodes * sizeof(S)) = f(q);
+  } else {
+    const rsrc_t r = rsrc(st + (uint64_t)(uint32_t)z * (uint32_t)p.ps, kAnyByte);
+    keep_here(off);
+#pragma unroll
+    for (int q = 0; q < NIL; q++) bst<2>(r, off + q * kRowNodes * (uint32_t)sizeof(S), f(q));
+  }
+}
 // Reduced storage: the raw values of one source, loaded before any is
 // converted (left to itself the scheduler reuses one register per load and
-// waits out each round trip).
+// waits out each round trip).  phi (psi) of the two component models comes
+// from the fused pass's LDS ring instead.
 template <int NC, typename S>
 struct RawSrc {
-  S v[10];
+  S v[NIL];
 };
-template <int NC, typename S>
-__device__ __forceinline__ void load_raw(const PlaneSrc &ps, uint32_t offS, RawSrc<NC, S> &r) {
-#pragma unroll
-  for (int q = 0; q < 10; q++) r.v[q] = bld<S>(rsrc(ps.f + q * ps.fsS, ps.pbS), offS);
-}
 template <int NC, typename S, bool CLO>
 __device__ __forceinline__ void convert_raw(const RawSrc<NC, S> &r, const Params &p, Src<NC, CLO> &s) {
 #pragma unroll
-  for (int q = 0; q < 10; q++) s.m[q] = dec(r.v[q], p, sgrp(q));
-}
-
-// FP32 storage: the moments of one source straight into place.
-template <int NC, bool CLO>
-__device__ __forceinline__ void load_m32(const PlaneSrc &ps, uint32_t offS, Src<NC, CLO> &s) {
-#pragma unroll
-  for (int q = 0; q < 10; q++) s.m[q] = bld<float>(rsrc(ps.f + q * ps.fsS, ps.pbS), offS);
+  for (int q = 0; q < NIL; q++) s.m[q] = dec(r.v[q], p, sgrp(q));
 }
 
 // The other loads of one source: gated curvature, closure.
@@ -932,7 +1042,7 @@ __device__ __forceinline__ ColourNode colour_node(const float *m, float gx, floa
   return c;
 }
 
-template <int NC, bool ADD, bool CLO, typename Sink>
+template <int NC, bool ADD, A2Form A2, bool CLO, typename Sink>
 __device__ __forceinline__ void eval_src(const Src<NC, CLO> &s, const Params &p, Sink &h, float *gq) {
   const float *m = s.m;
   float cbuf[10], om1;
@@ -947,7 +1057,7 @@ __device__ __forceinline__ void eval_src(const Src<NC, CLO> &s, const Params &p,
     const float esx = sx + p.fx + p.lin_a * m[1];
     const float esy = sy + p.fy + p.lin_a * m[2];
     const float esz = sz + p.fz + p.lin_a * m[3];
-    all_pops_mt<false>(mc, m[1] + esx, m[2] + esy, m[3] + esz, p, h, om1);
+    all_pops_mt<false, A2>(mc, m[1] + esx, m[2] + esy, m[3] + esz, p, h, om1);
     // D3Q7 phase field with sharpening, recursive_2c_TSLB3D.f90:808-831
     // g_{+-a} = phi/8 +- A_a with A_a = (3/8) phi u_a + sh n_a: the sink gets
     // A_x and A_y (the destination adds phi/8 of the source from the phi
@@ -971,7 +1081,7 @@ __device__ __forceinline__ void eval_src(const Src<NC, CLO> &s, const Params &p,
     const float gx = s.nn[0], gy = s.nn[1], gz = s.nn[2];
     const ColourNode c = colour_node(m, gx, gy, gz, p);
     ColourSink<Sink> cs(h, c.K, gx, gy, gz, c.g2);
-    all_pops_mt<ADD>(m, m[1], m[2], m[3], p, cs, 1.f - c.omega);
+    all_pops_mt<ADD, A2>(m, m[1], m[2], m[3], p, cs, 1.f - c.omega);
     gq[0] = c.ca;
     gq[1] = c.bc;
     gq[2] = gx;
@@ -979,10 +1089,10 @@ __device__ __forceinline__ void eval_src(const Src<NC, CLO> &s, const Params &p,
     gq[4] = gz;
   } else {
     if (p.shift) {
-      all_pops_mt<false>(mc, m[1] + (p.fx + p.lin_a * m[1]), m[2] + (p.fy + p.lin_a * m[2]),
+      all_pops_mt<false, A2>(mc, m[1] + (p.fx + p.lin_a * m[1]), m[2] + (p.fy + p.lin_a * m[2]),
                          m[3] + (p.fz + p.lin_a * m[3]), p, h, om1);
     } else {
-      all_pops_mt<ADD>(mc, m[1], m[2], m[3], p, h, om1);
+      all_pops_mt<ADD, A2>(mc, m[1], m[2], m[3], p, h, om1);
     }
   }
 }
@@ -990,7 +1100,7 @@ __device__ __forceinline__ void eval_src(const Src<NC, CLO> &s, const Params &p,
 // A ring source (one- and two-component models): eval_src restricted to the
 // 9 populations entering the tile (ring_pops) and, for the phase field, the
 // flux A_P along the side's normal axis (rf: LDS slot 24 for A_x, 25 for A_y).
-template <int NC, bool ADD, bool CLO>
+template <int NC, bool ADD, A2Form A2, bool CLO>
 __device__ __forceinline__ void eval_ring(const Src<NC, CLO> &s, const Params &p, bool col, float sgn,
                                           float *const (&rq)[3], float *rf) {
   const float *m = s.m;
@@ -1002,7 +1112,7 @@ __device__ __forceinline__ void eval_ring(const Src<NC, CLO> &s, const Params &p
     const float gx = s.nn[0], gy = s.nn[1], gz = s.nn[2];
     const ColourNode c = colour_node(m, gx, gy, gz, p);
     const ColourRingAdj adj{RingDir{col, sgn, gx, gy, gz}, c.K, c.g2};
-    ring_pops<ADD>(m, m[1], m[2], m[3], p, 1.f - c.omega, col, sgn, rq, adj);
+    ring_pops<ADD, A2>(m, m[1], m[2], m[3], p, 1.f - c.omega, col, sgn, rq, adj);
     rf[0] = c.ca;
     rf[1] = c.bc;
     rf[2] = gx;
@@ -1016,16 +1126,16 @@ __device__ __forceinline__ void eval_ring(const Src<NC, CLO> &s, const Params &p
     const float esx = sx + p.fx + p.lin_a * m[1];
     const float esy = sy + p.fy + p.lin_a * m[2];
     const float esz = sz + p.fz + p.lin_a * m[3];
-    ring_pops<false>(mc, m[1] + esx, m[2] + esy, m[3] + esz, p, om1, col, sgn, rq);
+    ring_pops<false, A2>(mc, m[1] + esx, m[2] + esy, m[3] + esz, p, om1, col, sgn, rq);
     const float sh = 0.125f * p.sharp_c * phi * (1.f - phi);
     const float base = 0.125f * phi;
     *rf = fmaf(3.f * base, col ? m[1] : m[2], sh * (col ? n0 : n1));
   } else {
     if (p.shift) {
-      ring_pops<false>(mc, m[1] + (p.fx + p.lin_a * m[1]), m[2] + (p.fy + p.lin_a * m[2]),
+      ring_pops<false, A2>(mc, m[1] + (p.fx + p.lin_a * m[1]), m[2] + (p.fy + p.lin_a * m[2]),
                        m[3] + (p.fz + p.lin_a * m[3]), p, om1, col, sgn, rq);
     } else {
-      ring_pops<ADD>(mc, m[1], m[2], m[3], p, om1, col, sgn, rq);
+      ring_pops<ADD, A2>(mc, m[1], m[2], m[3], p, om1, col, sgn, rq);
     }
   }
 }
@@ -1278,13 +1388,18 @@ __device__ __forceinline__ void append_runs(const uint64_t *wm, int *sbase, int 
   }
 }
 
-template <int NC, bool MASK, bool ADD, int WPE, typename S, bool CLO = false, bool R9 = true>
-__global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(WPE, 8))) void k_fused(
+// WIDE: 64-bit addresses, for planes of 4 GiB and more (see load_node)
+template <int NC, bool MASK, bool ADD, typename S, bool CLO = false, bool WIDE = false>
+__global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_fused(
     const S *__restrict__ src, S *__restrict__ dst, const float *__restrict__ nrm,
     const uint8_t *__restrict__ flags, const uint32_t *__restrict__ links, const float *__restrict__ clo,
     int *__restrict__ ilist, uint8_t *__restrict__ flags_next, Params p) {
   constexpr int NQ = NC == 2 ? 26 : 24;
   constexpr int NF = NC >= 2 ? 11 : 10;
+  // form of the off-diagonal a2 of own and ring sources
+  constexpr bool FX16 = std::is_same<S, fx16_t>::value;
+  constexpr A2Form A2_OWN = !CLO && (NC >= 2 || (FX16 && !ADD)) ? A2_PXY : A2_VV;
+  constexpr A2Form A2_RING = !CLO && (NC >= 2 || !FX16 || !ADD) ? A2_PXY : A2_VV;
   __shared__ float lds[NQ][NSLOT];
   // phase field: phi planes zs-1, zs, zs+1 of the (TX+4)x(TY+4) footprint
   constexpr int NPR = NC >= 2 ? 3 : 1;
@@ -1307,7 +1422,9 @@ __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(WPE, 8))) 
   const size_t plane = (size_t)p.nx * p.ny;
   const size_t tiles_plane = (size_t)p.tiles_x * p.tiles_y;
   const uint32_t pbS = (uint32_t)(plane * sizeof(S)), pb4 = (uint32_t)(plane * 4);
-  const long long fsS = p.fs * (long long)sizeof(S), fs4 = p.fs * 4;
+  const long long fs4 = p.fs * 4;
+  const S *const src_phi = src + p.phi0;
+  S *const dst_phi = dst + p.phi0;
 
   // own source column
   int ox = 0, oy = 0;
@@ -1337,7 +1454,9 @@ __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(WPE, 8))) 
                    src_coord(y0 + rsy - 1, p.ny, p.py, ry);
   // in-plane element offsets (loop-invariant) and flag tiles of both columns
   const uint32_t o_xy = (uint32_t)(ox + p.nx * oy), r_xy = (uint32_t)(rx + p.nx * ry);
-  const uint32_t d_xy = active ? (uint32_t)(x + p.nx * y) : 0u;
+  // byte offsets of both columns in the moment layout (an active node's source
+  // is the node itself, so o_xy and o_off are its destination's too)
+  const lane_off_t<WIDE> o_off = lane_off<S, WIDE>(p, ox, oy), r_off = lane_off<S, WIDE>(p, rx, ry);
   // curvature flag bytes of both source columns: one per half-tile
   const int o_tile = 2 * ((oy / TY) * p.tiles_x + ox / TX) + (ox % TX) / HX;
   const int r_tile = 2 * ((ry / TY) * p.tiles_x + rx / TX) + (rx % TX) / HX;
@@ -1353,7 +1472,7 @@ __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(WPE, 8))) 
   const uint32_t pofs0 = NC >= 2 ? phi_off(tid) : 0u, pofs1 = ptwo ? phi_off(tid + NTHR) : 0u;
   S pr0{}, pr1{};  // raw storage values, converted at commit
   auto phi_issue = [&](int z) {
-    const rsrc_t r = rsrc((const char *)src + TSLB_PHI * fsS + (size_t)clampw(z, p.nz, p.pz) * pbS, pbS);
+    const rsrc_t r = rsrc((const char *)src_phi + (size_t)clampw(z, p.nz, p.pz) * pbS, pbS);
     pr0 = bld<S>(r, pofs0);
     if (ptwo) pr1 = bld<S>(r, pofs1);
   };
@@ -1384,37 +1503,34 @@ __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(WPE, 8))) 
       if (z == p.nz - 1) m |= dirmask(2, -1);
     }
     if constexpr (MASK) {
-      if (active && z >= 0 && z < p.nz) m |= bld_u32(rsrc(links + plane * z, pb4), d_xy * 4u);
+      if (active && z >= 0 && z < p.nz) m |= bld_u32(rsrc(links + plane * z, pb4), o_xy * 4u);
     }
     return m;
   };
 
   // source fetch of one plane: own column and (tid < NRING) the ring slot
-  auto fetch = [&](int zs, Src<NC, CLO> &o, bool &ook, Src<NC, CLO> &r, bool &rok) {
+  auto fetch = [&](int zs, Src<NC, CLO> &o, bool &ook, Src<NC, CLO> &r, bool &rok, RawSrc<NC, S> &rwr) {
     int gz = 0;
     const bool zok = src_coord(zs, p.nz, p.pz, gz);
     PlaneSrc ps;
-    ps.f = (const char *)src + (size_t)gz * pbS;
     ps.n = (const char *)nrm + (size_t)gz * pb4;
     ps.c = (const char *)clo + (size_t)gz * pb4;
-    ps.pbS = pbS;
     ps.pb4 = pb4;
-    ps.fsS = fsS;
     ps.fs4 = fs4;
     const rsrc_t fl = rsrc(flags + 2 * tiles_plane * (size_t)gz, (uint32_t)(2 * tiles_plane));
     const rsrc_t lk = rsrc(links + plane * (size_t)gz, pb4);
     // Per source: link mask, curvature flag, moments, the flag-dependent
     // loads.  (Issuing both sources' masks and flags ahead of all moments
     // measured slower: 3.10 against 3.00 ms for 2C FP32.)
-    RawSrc<NC, S> rwo, rwr;  // reduced storage: converted after all loads
+    RawSrc<NC, S> rwo;  // reduced storage: converted after all loads, the ring's when it is evaluated
     ook = zok && oxy;
     if (ook) {
       if constexpr (MASK) ook = (bld_u32(lk, o_xy * 4u) & kSolid) == 0u;
       bool un = NC != 2;  // flags gate the phase-field curvature only
       if constexpr (NC == 2) un = bld_u8(fl, (uint32_t)o_tile) != 0;
       if (ook) {
-        if constexpr (sizeof(S) == 4) load_m32(ps, o_xy * 4u, o);
-        else load_raw<NC, S>(ps, o_xy * (uint32_t)sizeof(S), rwo);
+        load_node<S, WIDE>(src, p, gz, o_off, rwo.v);
+        if constexpr (sizeof(S) == 4) convert_raw(rwo, p, o);
         load_extra(ps, un ? o_xy * 4u : kOOB, o_xy * 4u, o);
       }
     }
@@ -1424,15 +1540,14 @@ __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(WPE, 8))) 
       bool un = NC != 2;
       if constexpr (NC == 2) un = bld_u8(fl, (uint32_t)r_tile) != 0;
       if (rok) {
-        if constexpr (sizeof(S) == 4) load_m32(ps, r_xy * 4u, r);
-        else load_raw<NC, S>(ps, r_xy * (uint32_t)sizeof(S), rwr);
+        load_node<S, WIDE>(src, p, gz, r_off, rwr.v);
+        if constexpr (sizeof(S) == 4) convert_raw(rwr, p, r);
         load_extra(ps, un ? r_xy * 4u : kOOB, r_xy * 4u, r);
       }
     }
     if constexpr (sizeof(S) != 4) {
       __builtin_amdgcn_sched_barrier(0);
       if (ook) convert_raw(rwo, p, o);
-      if (rok) convert_raw(rwr, p, r);
     }
   };
 
@@ -1453,6 +1568,7 @@ __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(WPE, 8))) 
     }
     Src<NC, CLO> co, cr;
     bool co_ok, cr_ok;
+    RawSrc<NC, S> cr_raw;
     // two-component models in FP32 storage: the plane's loads issue at raised
     // wave priority, ahead of the other block's arithmetic, so that their
     // latency starts counting early (2C emulsion 2.66 -> 2.63 ms, colour
@@ -1463,7 +1579,7 @@ __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(WPE, 8))) 
     // BF16 2.75 -> 2.62 ms; channel BF16 0.58 -> 0.54 ms); the colour model
     // keeps both (FP16 sphere 0.459 -> 0.448 ms with them)
     if constexpr (NC >= 2 && (sizeof(S) == 4 || NC == 3)) __builtin_amdgcn_s_setprio(2);
-    fetch(zs, co, co_ok, cr, cr_ok);
+    fetch(zs, co, co_ok, cr, cr_ok, cr_raw);
     // the waves that also evaluate ring sources keep priority 1 until the
     // barrier (they set when it releases), the others drop to 0
     const bool ring_wave = (tid >> 6) < (NRING + 63) / 64;
@@ -1488,7 +1604,7 @@ __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(WPE, 8))) 
         co.m[NF - 1] = p0[co_c];
       }
       PopSink sk{lds, (ty + 1) * SW + (tx + 1), 0.f, 0.f, 0.f};
-      eval_src<NC, ADD>(co, p, sk, gq);
+      eval_src<NC, ADD, A2_OWN>(co, p, sk, gq);
       h0 = sk.h0;
       h5 = sk.h5;
       h6 = sk.h6;
@@ -1505,27 +1621,23 @@ __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(WPE, 8))) 
     }
     // ---- halo ring slot
     if (cr_ok) {
+      if constexpr (sizeof(S) != 4) {
+        convert_raw(cr_raw, p, cr);
+      }
       if constexpr (NC >= 2) {
         cr.nn[0] = nnr[0];
         cr.nn[1] = nnr[1];
         cr.nn[2] = nnr[2];
         cr.m[NF - 1] = p0[cr_c];
       }
-      if constexpr (R9) {
-        // the 9 populations (and the phase flux, or the colour model's
-        // recolouring inputs) that enter the tile
-        bool col;
-        float sgn;
-        float *rq[3];
-        ring_geom(col, sgn, rq);
-        if constexpr (NC == 3) eval_ring<NC, ADD>(cr, p, col, sgn, rq, rc);
-        else eval_ring<NC, ADD>(cr, p, col, sgn, rq, &lds[col ? 24 : 25][rsy * SW + rsx]);
-      } else {
-        PopSink sk{lds, rsy * SW + rsx, 0.f, 0.f, 0.f};
-        eval_src<NC, ADD>(cr, p, sk, gq);
-        if constexpr (NC == 3)
-          for (int k = 0; k < 5; k++) rc[k] = gq[k];
-      }
+      // the 9 populations (and the phase flux, or the colour model's
+      // recolouring inputs) that enter the tile
+      bool col;
+      float sgn;
+      float *rq[3];
+      ring_geom(col, sgn, rq);
+      if constexpr (NC == 3) eval_ring<NC, ADD, A2_RING>(cr, p, col, sgn, rq, rc);
+      else eval_ring<NC, ADD, A2_RING>(cr, p, col, sgn, rq, &lds[col ? 24 : 25][rsy * SW + rsx]);
     }
     __builtin_amdgcn_s_setprio(0);
     __syncthreads();
@@ -1587,15 +1699,11 @@ __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(WPE, 8))) 
         a6 = ro.a<6>(h6);
       }
       if (cr_ok) {
-        if constexpr (R9) {
-          bool col;
-          float sgn;
-          float *rq[3];
-          ring_geom(col, sgn, rq);
-          colour_rewrite_ring(rq, rc, col, sgn);
-        } else {
-          colour_rewrite<1>(lds, rsy * SW + rsx, Recolour(rc));
-        }
+        bool col;
+        float sgn;
+        float *rq[3];
+        ring_geom(col, sgn, rq);
+        colour_rewrite_ring(rq, rc, col, sgn);
       }
       __builtin_amdgcn_s_setprio(0);
       __syncthreads();
@@ -1619,16 +1727,20 @@ __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(WPE, 8))) 
     const int zd = zs - 1;
     bool hit = false;  // phase field: may the new plane carry curvature here?
     if (active && zd >= z0 && zd < z1) {
-      const size_t zb = (size_t)zd * pbS;
-      const uint32_t offS = d_xy * (uint32_t)sizeof(S);
+      const rsrc_t dphi = rsrc((char *)dst_phi + (size_t)zd * pbS, pbS);
+      const uint32_t offS = o_xy * (uint32_t)sizeof(S);
+      auto put = [&](auto &&f) { store_node<S, WIDE>(dst, p, zd, o_off, f); };
       if (MASK && (bmA & kSolid)) {
-#pragma unroll
-        for (int q = 0; q < NF; q++)
-          bst<2>(rsrc((char *)dst + zb + q * fsS, pbS), offS,
-              bld<S>(rsrc((const char *)src + zb + q * fsS, pbS), offS));
-        if constexpr (NC == 2) {
-          const float f = dec(bld<S>(rsrc((const char *)src + zb + TSLB_PHI * fsS, pbS), offS), p, sgrp(TSLB_PHI));
-          hit = f * (1.f - f) > 0.19f;
+        S keep[NIL];
+        load_node<S, WIDE>(src, p, zd, o_off, keep);
+        put([&](int q) { return keep[q]; });
+        if constexpr (NC >= 2) {
+          const S sp = bld<S>(rsrc((const char *)src_phi + (size_t)zd * pbS, pbS), offS);
+          bst<2>(dphi, offS, sp);
+          if constexpr (NC == 2) {
+            const float f = dec(sp, p, sgrp(TSLB_PHI));
+            hit = f * (1.f - f) > 0.19f;
+          }
         }
       } else {
         const float rho = 1.f + aA.s0;
@@ -1673,28 +1785,26 @@ __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(WPE, 8))) 
             for (int q = 0; q < NF; q++)
               x[q] = __builtin_amdgcn_fmed3f(x[q], -32767.f, dithered(q) ? 32766.f : 32767.f);
           }
-          const uint32_t h1 = node_hash(d_xy + (uint32_t)plane * (uint32_t)zd, p.step);
+          const uint32_t h1 = node_hash(o_xy + (uint32_t)plane * (uint32_t)zd, p.step);
           const uint32_t h2 = node_rehash(h1);
           const uint32_t w[5] = {h1 & 0xFFFFu, h1 >> 16, h2 & 0xFFFFu, h2 >> 16, (h1 ^ h2) & 0xFFFFu};
-#pragma unroll
-          for (int q = 0; q < NF; q++)
-            bst<2>(rsrc((char *)dst + zb + q * fsS, pbS), offS,
-                   dithered(q) ? fx16_dither(x[q], w[dither_word(q)]) : fx16_code(x[q]));
+          put([&](int q) { return dithered(q) ? fx16_dither(x[q], w[dither_word(q)]) : fx16_code(x[q]); });
+          if constexpr (NC >= 2) bst<2>(dphi, offS, fx16_dither(x[TSLB_PHI], w[dither_word(TSLB_PHI)]));
         } else if constexpr (sizeof(S) == 4) {
-#pragma unroll
-          for (int q = 0; q < NF; q++) bst<2>(rsrc((char *)dst + zb + q * fsS, pbS), offS, from_f<S>(out[q]));
+          put([&](int q) { return from_f<S>(out[q]); });
+          if constexpr (NC >= 2) bst<2>(dphi, offS, out[TSLB_PHI]);
         } else {
           // FP16, BF16: rho - 1, u, v, w and phi with stochastic rounding,
           // 32 random bits each
-          const uint32_t h1 = node_hash(d_xy + (uint32_t)plane * (uint32_t)zd, p.step);
+          const uint32_t h1 = node_hash(o_xy + (uint32_t)plane * (uint32_t)zd, p.step);
           const uint32_t h2 = node_rehash(h1);
           const uint32_t rw[5] = {h1, h2, rot16(h1), rot16(h2), h1 ^ h2};
-#pragma unroll
-          for (int q = 0; q < NF; q++) {
+          put([&](int q) {
             const float v = out[q] * p.sc[sgrp(q)];
-            bst<2>(rsrc((char *)dst + zb + q * fsS, pbS), offS,
-                   dithered(q) ? from_f_sr<S>(v, rw[dither_word(q)]) : from_f<S>(v));
-          }
+            return dithered(q) ? from_f_sr<S>(v, rw[dither_word(q)]) : from_f<S>(v);
+          });
+          if constexpr (NC >= 2)
+            bst<2>(dphi, offS, from_f_sr<S>(out[TSLB_PHI] * p.sc[sgrp(TSLB_PHI)], rw[dither_word(TSLB_PHI)]));
         }
         if constexpr (NC == 2) hit = out[10] * (1.f - out[10]) > 0.19f;
       }
@@ -2238,29 +2348,23 @@ __global__ __launch_bounds__(256) void k_copy(const v4f *__restrict__ a, v4f *__
 // invalid sources.
 // ---------------------------------------------------------------------------
 template <typename S>
-__global__ __launch_bounds__(256) void k_prepush(const S *__restrict__ phi,
-                                                 const S *__restrict__ u,
-                                                 const S *__restrict__ v,
-                                                 const S *__restrict__ w,
-                                                 S *__restrict__ out,
+__global__ __launch_bounds__(256) void k_prepush(const S *__restrict__ st, S *__restrict__ out,
                                                  const uint32_t *__restrict__ links, int has_mask,
                                                  Params p) {
   const int n = p.nx * p.ny * p.nz;
   const int id = blockIdx.x * 256 + threadIdx.x;
   if (id >= n) return;
+  const S *phi = st + p.phi0;
   if (has_mask && (links[id] & kSolid)) {
     out[id] = phi[id];
     return;
   }
-  const int x = id % p.nx;
-  const int y = (id / p.nx) % p.ny;
-  const int z = id / (p.nx * p.ny);
-  const S *vel[3] = {u, v, w};
+  const auto [x, y, z] = node_of(p, id);
   float own[7];
-  const float ph0 = ldf(phi, id, p, TSLB_PHI);
+  const float ph0 = ldv(phi, id, p, TSLB_PHI);
   own[0] = 0.25f * ph0;
   for (int a = 0; a < 3; a++) {
-    const float ua = ldf(vel[a], id, p, TSLB_U + a);
+    const float ua = ldf(st, TSLB_U + a, x, y, z, p);
     own[1 + 2 * a] = 0.125f * ph0 * (1.f + 3.f * ua);
     own[2 + 2 * a] = 0.125f * ph0 * (1.f - 3.f * ua);
   }
@@ -2276,10 +2380,10 @@ __global__ __launch_bounds__(256) void k_prepush(const S *__restrict__ phi,
     } else {
       const int a = (l - 1) / 2;
       const float sgn = (l & 1) ? 1.f : -1.f;
-      s += 0.125f * ldf(phi, sid, p, TSLB_PHI) * (1.f + sgn * 3.f * ldf(vel[a], sid, p, TSLB_U + a));
+      s += 0.125f * ldv(phi, sid, p, TSLB_PHI) * (1.f + sgn * 3.f * ldf(st, TSLB_U + a, sx, sy, sz, p));
     }
   }
-  stf(out, id, s, p, TSLB_PHI);
+  stv(out, id, s, p, TSLB_PHI);
 }
 
 // ---------------------------------------------------------------------------
@@ -2314,21 +2418,21 @@ __global__ __launch_bounds__(256) void k_links(const int32_t *__restrict__ isf,
 // plane 0 <- plane 1 with u = v = 0 and w = w_in; plane nz-1 <- plane nz-2.
 // ---------------------------------------------------------------------------
 template <typename S>
-__global__ __launch_bounds__(256) void k_zplane_bc(FieldsT<S> f, const float *__restrict__ w_in,
+__global__ __launch_bounds__(256) void k_zplane_bc(S *__restrict__ st, const float *__restrict__ w_in,
                                                    const float *__restrict__ phi_in, int ncomp,
                                                    Params p) {
   const int plane = p.nx * p.ny;
   const int id = blockIdx.x * 256 + threadIdx.x;
   if (id >= plane) return;
-  const int lo = id, lo1 = id + plane;
-  const int hi = id + plane * (p.nz - 1), hi1 = id + plane * (p.nz - 2);
+  const int x = id % p.nx, y = id / p.nx;
+  auto at = [&](int q, int z) -> S & { return st[mom_off<(int)sizeof(S)>(p, q, x, y, z)]; };
   const int nf = ncomp >= 2 ? TSLB_NFIELDS : 10;
-  for (int q = 0; q < nf; q++) f.f[q][hi] = f.f[q][hi1];
+  for (int q = 0; q < nf; q++) at(q, p.nz - 1) = at(q, p.nz - 2);
   for (int q = 0; q < nf; q++) {
-    if (q == TSLB_U || q == TSLB_V) stf(f.f[q], lo, 0.f, p, q);
-    else if (q == TSLB_W) stf(f.f[q], lo, w_in[id], p, q);
-    else if (q == TSLB_PHI && phi_in) stf(f.f[q], lo, phi_in[id], p, q);
-    else f.f[q][lo] = f.f[q][lo1];
+    if (q == TSLB_U || q == TSLB_V) stf(st, q, x, y, 0, 0.f, p);
+    else if (q == TSLB_W) stf(st, q, x, y, 0, w_in[id], p);
+    else if (q == TSLB_PHI && phi_in) stf(st, q, x, y, 0, phi_in[id], p);
+    else at(q, 0) = at(q, 1);
   }
 }
 
@@ -2361,10 +2465,10 @@ __global__ __launch_bounds__(256) void k_jet_bc(const S *__restrict__ src, S *__
   const int i = xy % p.nx, j = xy / p.nx;
   const int zy = side ? p.nz - 2 : 1, zx = side ? p.nz - 1 : 0;
   const int sz = side ? -1 : 1;  // c_z of the populations crossing into plane zy
-  auto at = [&](int q, int id) -> float { return ldf(src + (size_t)q * p.fs, id, p, q); };
+  auto at = [&](int q, int xx, int yy, int zz) -> float { return ldf(src, q, xx, yy, zz, p); };
   if (side) {
     // outlet wall plane: w(x) = w(x - e_z), boundary_cds_3D_module.f90:992
-    stf(dst + (size_t)TSLB_W * p.fs, xy + plane * zx, at(TSLB_W, xy + plane * zy), p, TSLB_W);
+    stf(dst, TSLB_W, i, j, zx, at(TSLB_W, i, j, zy), p);
   }
   const int y = xy + plane * zy;
   const uint32_t ly = links[y];
@@ -2374,7 +2478,7 @@ __global__ __launch_bounds__(256) void k_jet_bc(const S *__restrict__ src, S *__
   // evaluated them for the bounce-back
   Src<NC> sy;
 #pragma unroll
-  for (int q = 0; q < (NC == 2 ? 11 : 10); q++) sy.m[q] = at(q, y);
+  for (int q = 0; q < (NC == 2 ? 11 : 10); q++) sy.m[q] = at(q, i, j, zy);
   if constexpr (NC == 2) {
     // n from phi as the fused pass computes it; planes zy +- 1 are in range
     float ph3[3][9];
@@ -2385,7 +2489,7 @@ __global__ __launch_bounds__(256) void k_jet_bc(const S *__restrict__ src, S *__
 #pragma unroll
         for (int dx = -1; dx <= 1; dx++) {
           const int gi = clampw(i + dx, p.nx, p.px), gj = clampw(j + dy, p.ny, p.py);
-          ph3[dz + 1][(dy + 1) * 3 + dx + 1] = at(TSLB_PHI, gi + p.nx * gj + plane * (zy + dz));
+          ph3[dz + 1][(dy + 1) * 3 + dx + 1] = at(TSLB_PHI, gi, gj, zy + dz);
         }
     sep_normal<3>(ph3[0], ph3[1], ph3[2], 4, sy.nn[0], sy.nn[1], sy.nn[2]);
     const int tile = (j / TY) * p.tiles_x + i / TX;
@@ -2394,10 +2498,10 @@ __global__ __launch_bounds__(256) void k_jet_bc(const S *__restrict__ src, S *__
   }
   ArraySink own;
   float gq[7];
-  eval_src<NC, ADD>(sy, p, own, gq);
+  eval_src<NC, ADD, ADD ? A2_VV : A2_SUM>(sy, p, own, gq);
 
   // shifted sums of y from its finished moments
-  auto dat = [&](int q) -> float { return ldf(dst + (size_t)q * p.fs, y, p, q); };
+  auto dat = [&](int q) -> float { return ldf(dst, q, i, j, zy, p); };
   const float s0 = dat(TSLB_RHO), rho = 1.f + s0;
   const float u1 = dat(TSLB_U), v1 = dat(TSLB_V), w1 = dat(TSLB_W);
   const float t3 = s0 * (1.f / 3.f);
@@ -2417,11 +2521,10 @@ __global__ __launch_bounds__(256) void k_jet_bc(const S *__restrict__ src, S *__
     if (kCZ[l] != sz || !((ly >> l) & 1u)) continue;
     int xi = 0, xj = 0;
     if (!src_coord(i - kCX[l], p.nx, p.px, xi) || !src_coord(j - kCY[l], p.ny, p.py, xj)) continue;
-    const int x = xi + p.nx * xj + plane * zx;
-    const float ux = at(TSLB_U, x), vx = at(TSLB_V, x);
-    const float wx = side ? at(TSLB_W, xi + p.nx * xj + plane * zy) : at(TSLB_W, x);
+    const float ux = at(TSLB_U, xi, xj, zx), vx = at(TSLB_V, xi, xj, zx);
+    const float wx = at(TSLB_W, xi, xj, side ? zy : zx);
     ArraySink bnd;
-    all_pops_mt<false>(sy.m, ux, vx, wx, p, bnd, p.om1);
+    all_pops_mt<false, A2_VV>(sy.m, ux, vx, wx, p, bnd, p.om1);
     const float d = bnd.h[l] - own.h[kOPP[l]];
     const float cx = (float)kCX[l], cy = (float)kCY[l], cz = (float)kCZ[l];
     sm[0] += d;
@@ -2444,17 +2547,16 @@ __global__ __launch_bounds__(256) void k_jet_bc(const S *__restrict__ src, S *__
     const float out[10] = {sm[0], u, v, w, sm[4] - tt - r * u * u, sm[5] - tt - r * v * v,
                            sm[6] - tt - r * w * w, sm[7] - r * u * v, sm[8] - r * u * w, sm[9] - r * v * w};
 #pragma unroll
-    for (int q = 0; q < 10; q++) stf(dst + (size_t)q * p.fs, y, out[q], p, q);
+    for (int q = 0; q < 10; q++) stf(dst, q, i, j, zy, out[q], p);
   }
   if constexpr (NC == 2) {
     float add;
     if (!side) {
-      const int x = xy + plane * zx;
-      add = 0.125f * at(TSLB_PHI, x) * (1.f + 3.f * at(TSLB_W, x));
+      add = 0.125f * at(TSLB_PHI, i, j, zx) * (1.f + 3.f * at(TSLB_W, i, j, zx));
     } else {
       add = 0.125f * sy.m[TSLB_PHI] * (1.f - 3.f * 0.05f);
     }
-    stf(dst + (size_t)TSLB_PHI * p.fs, y, dat(TSLB_PHI) + add, p, TSLB_PHI);
+    stf(dst, TSLB_PHI, i, j, zy, dat(TSLB_PHI) + add, p);
   }
 }
 
@@ -2494,37 +2596,65 @@ __host__ __device__ inline float rand_noseeded_impl(int i, int j, int k, int l) 
 // field += amp * (2 r - 1), r = rand_noseeded(i, j, k, l) with 1-based i, j, k
 // (seeding as TSLB_2C-mpi/lb_kernels_module.f90:970-977)
 template <typename S>
-__global__ __launch_bounds__(256) void k_seed_noise(S *__restrict__ a, int q, float amp, int l, Params p) {
+__global__ __launch_bounds__(256) void k_seed_noise(S *__restrict__ st, int q, float amp, int l, Params p) {
   const int n = p.nx * p.ny * p.nz;
   const int id = blockIdx.x * 256 + threadIdx.x;
   if (id >= n) return;
-  const int x = id % p.nx;
-  const int y = (id / p.nx) % p.ny;
-  const int z = id / (p.nx * p.ny);
+  const auto [x, y, z] = node_of(p, id);
   const float r = rand_noseeded_impl(x + 1, y + 1, z + 1, l);
-  stf(a, id, ldf(a, id, p, q) + amp * (2.0f * r - 1.0f), p, q);
+  const uint64_t o = mom_off<(int)sizeof(S)>(p, q, x, y, z);
+  stv(st, o, ldv(st, o, p, q) + amp * (2.0f * r - 1.0f), p, q);
 }
 
-// host-format float <-> storage, with the field's scale; field 0 carries rho-1
+// host-format float <-> storage of field q at the nodes id0 .. id0 + n - 1,
+// with the field's scale; field 0 carries rho-1
 template <typename S>
-__global__ __launch_bounds__(256) void k_to_storage(const float *__restrict__ in, S *__restrict__ out,
-                                                    int n, int q, Params p) {
-  const int id = blockIdx.x * 256 + threadIdx.x;
-  if (id >= n) return;
-  const float v = q == TSLB_RHO ? in[id] - 1.0f : in[id];
-  stf(out, id, v, p, q);
+__global__ __launch_bounds__(256) void k_to_storage(const float *__restrict__ in, S *__restrict__ st,
+                                                    int id0, int n, int q, Params p) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= n) return;
+  const auto [x, y, z] = node_of(p, id0 + i);
+  stf(st, q, x, y, z, q == TSLB_RHO ? in[i] - 1.0f : in[i], p);
 }
 template <typename S>
-__global__ __launch_bounds__(256) void k_from_storage(const S *__restrict__ in, float *__restrict__ out,
+__global__ __launch_bounds__(256) void k_from_storage(const S *__restrict__ st, float *__restrict__ out,
                                                       int n, int q, Params p) {
   const int id = blockIdx.x * 256 + threadIdx.x;
   if (id >= n) return;
-  const float v = ldf(in, id, p, q);
+  const auto [x, y, z] = node_of(p, id);
+  const float v = ldf(st, q, x, y, z, p);
   out[id] = q == TSLB_RHO ? 1.0f + v : v;
 }
-
-__global__ __launch_bounds__(256) void k_fill(float *__restrict__ a, float v, int n) {
+// the stored values of field q, verbatim, in node order (checkpoints)
+template <typename S>
+__global__ __launch_bounds__(256) void k_pack_field(const S *__restrict__ st, S *__restrict__ out, int n, int q,
+                                                    Params p) {
   const int id = blockIdx.x * 256 + threadIdx.x;
+  if (id >= n) return;
+  const auto [x, y, z] = node_of(p, id);
+  out[id] = st[mom_off<(int)sizeof(S)>(p, q, x, y, z)];
+}
+template <typename S>
+__global__ __launch_bounds__(256) void k_unpack_field(const S *__restrict__ in, S *__restrict__ st, int n, int q,
+                                                      Params p) {
+  const int id = blockIdx.x * 256 + threadIdx.x;
+  if (id >= n) return;
+  const auto [x, y, z] = node_of(p, id);
+  st[mom_off<(int)sizeof(S)>(p, q, x, y, z)] = in[id];
+}
+// Pi^neq = 0 at every node (all-zero bits in every storage type)
+template <typename S>
+__global__ __launch_bounds__(256) void k_zero_pi(S *__restrict__ st, int n, Params p) {
+  const int id = blockIdx.x * 256 + threadIdx.x;
+  if (id >= n) return;
+  const auto [x, y, z] = node_of(p, id);
+  const uint64_t o = mom_off<(int)sizeof(S)>(p, TSLB_PXX, x, y, z);
+#pragma unroll
+  for (int q = 0; q < 6; q++) st[o + q * kRowNodes] = S{};
+}
+
+__global__ __launch_bounds__(256) void k_fill(float *__restrict__ a, float v, long long n) {
+  const long long id = blockIdx.x * 256LL + threadIdx.x;
   if (id < n) a[id] = v;
 }
 
@@ -2535,7 +2665,7 @@ __global__ __launch_bounds__(256) void k_fill(float *__restrict__ a, float v, in
 // ---------------------------------------------------------------------------
 constexpr int NRED = 7;
 template <typename S>
-__global__ __launch_bounds__(256) void k_reduce_part(CFieldsT<S> f, const uint32_t *__restrict__ links,
+__global__ __launch_bounds__(256) void k_reduce_part(const S *__restrict__ st, const uint32_t *__restrict__ links,
                                                      int has_mask, Params p,
                                                      double *__restrict__ part) {
   __shared__ double sh[NRED][256];
@@ -2543,28 +2673,30 @@ __global__ __launch_bounds__(256) void k_reduce_part(CFieldsT<S> f, const uint32
   double acc[NRED] = {0, 0, 0, 0, 0, 0, 0};
   for (int id = blockIdx.x * 256 + threadIdx.x; id < n; id += gridDim.x * 256) {
     if (has_mask && (links[id] & kSolid)) continue;
-    const int x = id % p.nx;
-    const int y = (id / p.nx) % p.ny;
-    const int z = id / (p.nx * p.ny);
-    const double rho = 1.0 + (double)ldf(f.f[0], id, p, 0);
-    const double u = ldf(f.f[1], id, p, 1), v = ldf(f.f[2], id, p, 2), w = ldf(f.f[3], id, p, 3);
+    const auto [x, y, z] = node_of(p, id);
+    // a node's offset is its column's and its plane's: five columns and three
+    // planes give the 13 nodes of the curl
+    auto side = [](int a, int n, int per) { return a < 0 ? (per ? n - 1 : 0) : (a < n ? a : (per ? 0 : n - 1)); };
+    auto col = [&](int xx, int yy) { return node_off<(int)sizeof(S)>(p, xx, yy); };
+    const uint64_t c0 = col(x, y), cxm = col(side(x - 1, p.nx, p.px), y), cxp = col(side(x + 1, p.nx, p.px), y);
+    const uint64_t cym = col(x, side(y - 1, p.ny, p.py)), cyp = col(x, side(y + 1, p.ny, p.py));
+    const uint64_t z0 = plane_off(p, z), zm = plane_off(p, side(z - 1, p.nz, p.pz)),
+                   zp = plane_off(p, side(z + 1, p.nz, p.pz));
+    auto at = [&](int q, uint64_t plane, uint64_t column) -> double {
+      return (double)ldv(st, plane + column + (uint32_t)(q * kRowNodes), p, q);
+    };
+    const double rho = 1.0 + at(0, z0, c0);
+    const double u = at(1, z0, c0), v = at(2, z0, c0), w = at(3, z0, c0);
     acc[0] += rho;
-    if (p.ncomp == 2) acc[1] += (double)ldf(f.f[TSLB_PHI], id, p, TSLB_PHI);
-    if (p.ncomp == TSLB_COLOUR) acc[1] += 0.5 * rho * (1.0 + (double)ldf(f.f[TSLB_PHI], id, p, TSLB_PHI));
+    if (p.ncomp == 2) acc[1] += (double)ldv(st, p.phi0 + id, p, TSLB_PHI);
+    if (p.ncomp == TSLB_COLOUR) acc[1] += 0.5 * rho * (1.0 + (double)ldv(st, p.phi0 + id, p, TSLB_PHI));
     acc[2] += 0.5 * rho * (u * u + v * v + w * w);
     acc[3] += rho * u;
     acc[4] += rho * v;
     acc[5] += rho * w;
-    auto at = [&](int q, int dx, int dy, int dz) -> double {
-      int xx = x + dx, yy = y + dy, zz = z + dz;
-      if (xx < 0 || xx >= p.nx) xx = p.px ? wrapc(xx, p.nx) : (xx < 0 ? 0 : p.nx - 1);
-      if (yy < 0 || yy >= p.ny) yy = p.py ? wrapc(yy, p.ny) : (yy < 0 ? 0 : p.ny - 1);
-      if (zz < 0 || zz >= p.nz) zz = p.pz ? wrapc(zz, p.nz) : (zz < 0 ? 0 : p.nz - 1);
-      return (double)ldf(f.f[q], xx + p.nx * yy + p.nx * p.ny * zz, p, q);
-    };
-    const double wx = 0.5 * (at(3, 0, 1, 0) - at(3, 0, -1, 0)) - 0.5 * (at(2, 0, 0, 1) - at(2, 0, 0, -1));
-    const double wy = 0.5 * (at(1, 0, 0, 1) - at(1, 0, 0, -1)) - 0.5 * (at(3, 1, 0, 0) - at(3, -1, 0, 0));
-    const double wz = 0.5 * (at(2, 1, 0, 0) - at(2, -1, 0, 0)) - 0.5 * (at(1, 0, 1, 0) - at(1, 0, -1, 0));
+    const double wx = 0.5 * (at(3, z0, cyp) - at(3, z0, cym)) - 0.5 * (at(2, zp, c0) - at(2, zm, c0));
+    const double wy = 0.5 * (at(1, zp, c0) - at(1, zm, c0)) - 0.5 * (at(3, z0, cxp) - at(3, z0, cxm));
+    const double wz = 0.5 * (at(2, z0, cxp) - at(2, z0, cxm)) - 0.5 * (at(1, z0, cyp) - at(1, z0, cym));
     acc[6] += 0.5 * (wx * wx + wy * wy + wz * wz);
   }
   for (int q = 0; q < NRED; q++) sh[q][threadIdx.x] = acc[q];
@@ -2648,8 +2780,9 @@ struct tslb_ctx {
   tslb_params prm;
   Params kp;
   hipStream_t stream = nullptr;
-  size_t n = 0, fs = 0;  // nodes, field stride (elements)
+  size_t n = 0, fs = 0;  // nodes, stride of the plain per-node arrays (elements)
   size_t es = 4;         // bytes per stored moment value
+  size_t len = 0;        // stored values of a state buffer (moment layout and phi)
   void *buf[2] = {nullptr, nullptr};
   int cur = 0;
   int phi_buf = 0;  // one component: the buffer that holds phi
@@ -2669,8 +2802,6 @@ struct tslb_ctx {
   int zbc = 0, zbc_phi = 0;
   int jet = 0;     // turbulent-jet inlet/outlet planes (k_jet_bc after k_fused)
   int zwalls = 0;  // bit 0: plane 0 all solid; bit 1: plane nz-1 all solid
-  int variant = 2;  // bit 1: cap VGPRs at 128 (two blocks per CU); bit 2: for comparisons, the
-                    // phase-field FP32 kernel with the full 27-population ring evaluation
   // learned closure: 0 none, 1 fixed per-node fields, 2 recomputed before
   // every collision by `model` from the current state
   int clo_mode = 0;
@@ -2724,21 +2855,10 @@ auto with_storage(const tslb_ctx *c, Fn &&fn) {
 }
 
 template <typename S>
-S *field_ptr(void *base, size_t fs, int q) {
-  return (S *)base + (size_t)q * fs;
+S *phi_ptr(const tslb_ctx *c, int b) {
+  return (S *)c->buf[b] + c->kp.phi0;
 }
-template <typename S>
-FieldsT<S> fields_of(void *base, size_t fs) {
-  FieldsT<S> f;
-  for (int q = 0; q < TSLB_NFIELDS; q++) f.f[q] = field_ptr<S>(base, fs, q);
-  return f;
-}
-template <typename S>
-CFieldsT<S> cfields_of(const void *base, size_t fs) {
-  CFieldsT<S> f;
-  for (int q = 0; q < TSLB_NFIELDS; q++) f.f[q] = (const S *)base + (size_t)q * fs;
-  return f;
-}
+unsigned grid_for(size_t n) { return (unsigned)((n + 255) / 256); }
 
 int dev_alloc(tslb_ctx *c, void **p, size_t bytes) {
   hipError_t e = hipMalloc(p, bytes);
@@ -2778,14 +2898,6 @@ int drain_timing(tslb_ctx *c) {
   return TSLB_OK;
 }
 
-// zero a field range of the state buffer (any storage type: all-zero bits)
-void zero_fields(tslb_ctx *c, void *base, int q0, int q1) {
-  const size_t words = (size_t)(q1 - q0) * c->fs * c->es / 4;
-  float *start = (float *)((char *)base + (size_t)q0 * c->fs * c->es);
-  hipLaunchKernelGGL(k_fill, dim3((unsigned)((words + 255) / 256)), dim3(256), 0, c->stream, start, 0.f,
-                     (int)words);
-}
-
 int launch_closure(tslb_ctx *c);  // closure_api.h
 
 int launch_normals(tslb_ctx *c, int dense = 0) {
@@ -2800,18 +2912,18 @@ int launch_normals(tslb_ctx *c, int dense = 0) {
     using S = decltype(tag);
     if (c->prm.ncomp == TSLB_COLOUR)
       hipLaunchKernelGGL((k_normals_tiled<S, true>), dim3(nblk), dim3(NTHR), 0, c->stream,
-                         field_ptr<S>(c->buf[c->cur], c->fs, TSLB_PHI), c->nrm, c->nrm + c->fs,
+                         phi_ptr<S>(c, c->cur), c->nrm, c->nrm + c->fs,
                          c->nrm + 2 * c->fs, c->nrm + 3 * c->fs, c->flags, c->links, c->has_mask, 1,
                          c->kp);
     else if (dense)
       hipLaunchKernelGGL((k_normals_tiled<S, false>), dim3(nblk), dim3(NTHR), 0, c->stream,
-                         field_ptr<S>(c->buf[c->cur], c->fs, TSLB_PHI), c->nrm, c->nrm + c->fs,
+                         phi_ptr<S>(c, c->cur), c->nrm, c->nrm + c->fs,
                          c->nrm + 2 * c->fs, c->nrm + 3 * c->fs, c->flags, c->links, c->has_mask,
                          1, c->kp);
     else {
       // sparse curvature: list the tile-planes that may carry it, then
       // compute those only
-      const S *phi = field_ptr<S>(c->buf[c->cur], c->fs, TSLB_PHI);
+      const S *phi = phi_ptr<S>(c, c->cur);
       if (!c->list_ok) {  // else the last fused pass listed the runs and cleared the flags
         hipLaunchKernelGGL(k_fill, dim3(1), dim3(256), 0, c->stream, (float *)c->ilist, 0.f, 1);
         hipLaunchKernelGGL((k_iface_list<S>), dim3(nblk), dim3(NTHR), 0, c->stream, phi, c->flags, c->ilist,
@@ -2841,7 +2953,6 @@ int launch_fused(tslb_ctx *c) {
     HIPCK(hipEventRecord(e0, c->stream));
   }
   const bool add = p.ncomp != 2 && !p.shift && (p.fx != 0.f || p.fy != 0.f || p.fz != 0.f);
-  const bool w4 = (c->variant & 2) != 0;
   // phase field: the fused pass lists the next step's interface runs unless
   // a boundary pass still changes phi after it
   const bool build = p.ncomp == 2 && !c->jet && !c->zbc;
@@ -2851,59 +2962,32 @@ int launch_fused(tslb_ctx *c) {
     using S = decltype(tag);
     const S *s = (const S *)c->buf[c->cur];
     S *d = (S *)c->buf[1 - c->cur];
-#define TSLB_LAUNCH(NC, MASK, ADD, WPE)                                                          \
-  do {                                                                                             \
-    if (c->clo_mode) {                                                                             \
-      if constexpr (NC != TSLB_COLOUR)                                                             \
-        hipLaunchKernelGGL((k_fused<NC, MASK, ADD, 4, S, true>), dim3(nblk), dim3(NTHR), 0,        \
-                           c->stream, s, d, c->nrm, c->flags, c->links, c->clo, ilist, c->flags_alt, p); \
-    } else {                                                                                       \
-      bool done = false;                                                                           \
-      if constexpr (NC == 2 && !MASK && WPE == 4 && sizeof(S) == 4) {                               \
-        if (c->variant & 4) {                                                                      \
-          hipLaunchKernelGGL((k_fused<NC, MASK, ADD, WPE, S, false, false>), dim3(nblk), dim3(NTHR), \
-                             0, c->stream, s, d, c->nrm, c->flags, c->links, (const float *)nullptr, \
-                             ilist, c->flags_alt, p);                                              \
-          done = true;                                                                             \
-        }                                                                                          \
-      }                                                                                            \
-      if (!done)                                                                                   \
-        hipLaunchKernelGGL((k_fused<NC, MASK, ADD, WPE, S>), dim3(nblk), dim3(NTHR), 0, c->stream,  \
-                           s, d, c->nrm, c->flags, c->links, (const float *)nullptr, ilist,        \
-                           c->flags_alt, p);                                                       \
-    }                                                                                              \
-  } while (0)
-    // FP32 storage keeps both register budgets selectable for sweeps (capped
-    // at 128 VGPRs for two blocks per CU, or uncapped); reduced storage is capped
-#define TSLB_LAUNCH_V(NC, MASK, ADD)                                      \
-  do {                                                                    \
-    if constexpr (sizeof(S) == 4) {                                       \
-      if (w4) TSLB_LAUNCH(NC, MASK, ADD, 4);                              \
-      else TSLB_LAUNCH(NC, MASK, ADD, 1);                                 \
-    } else {                                                              \
-      TSLB_LAUNCH(NC, MASK, ADD, 4);                                      \
-    }                                                                     \
-  } while (0)
-    if (p.ncomp == 2) {
-      if (c->has_mask) TSLB_LAUNCH_V(2, true, false);
-      else TSLB_LAUNCH_V(2, false, false);
+    auto go = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3(nblk), dim3(NTHR), 0, c->stream, s, d, c->nrm, c->flags, c->links, c->clo, ilist,
+                         c->flags_alt, p);
+    };
+    auto with_closure = [&](auto plain, auto closure) { c->clo_mode ? go(closure) : go(plain); };
+#define TSLB_KERNEL(NC, MASK, ADD) k_fused<NC, MASK, ADD, S>, k_fused<NC, MASK, ADD, S, true>
+    if (p.wide) {
+      // the general forms only: links are all fluid without a mask, a zero
+      // force adds nothing
+      if (p.ncomp == 2) with_closure(k_fused<2, true, false, S, false, true>, k_fused<2, true, false, S, true, true>);
+      else if (p.ncomp == TSLB_COLOUR) go(k_fused<3, true, true, S, false, true>);
+      else with_closure(k_fused<1, true, true, S, false, true>, k_fused<1, true, true, S, true, true>);
+    } else if (p.ncomp == 2) {
+      if (c->has_mask) with_closure(TSLB_KERNEL(2, true, false));
+      else with_closure(TSLB_KERNEL(2, false, false));
     } else if (p.ncomp == TSLB_COLOUR) {
-      if (c->has_mask) {
-        if (add) TSLB_LAUNCH_V(3, true, true);
-        else TSLB_LAUNCH_V(3, true, false);
-      } else {
-        if (add) TSLB_LAUNCH_V(3, false, true);
-        else TSLB_LAUNCH_V(3, false, false);
-      }
+      if (c->has_mask) add ? go(k_fused<3, true, true, S>) : go(k_fused<3, true, false, S>);
+      else add ? go(k_fused<3, false, true, S>) : go(k_fused<3, false, false, S>);
     } else if (add) {
-      if (c->has_mask) TSLB_LAUNCH_V(1, true, true);
-      else TSLB_LAUNCH_V(1, false, true);
+      if (c->has_mask) with_closure(TSLB_KERNEL(1, true, true));
+      else with_closure(TSLB_KERNEL(1, false, true));
     } else {
-      if (c->has_mask) TSLB_LAUNCH_V(1, true, false);
-      else TSLB_LAUNCH_V(1, false, false);
+      if (c->has_mask) with_closure(TSLB_KERNEL(1, true, false));
+      else with_closure(TSLB_KERNEL(1, false, false));
     }
-#undef TSLB_LAUNCH_V
-#undef TSLB_LAUNCH
+#undef TSLB_KERNEL
     return 0;
   });
   HIPCK(hipGetLastError());
@@ -2947,13 +3031,41 @@ int launch_fused(tslb_ctx *c) {
   return TSLB_OK;
 }
 
+// The moment layout of a lattice (see NIL above): tiles in superpages unless
+// the padding (partial tiles, a partial line of tiles) makes a buffer half as
+// large again; a buffer of up to 2^23 values (32 MiB in FP32) may be any
+// multiple of its nodes.
+// all nodes fluid, no links across solids (the wide kernels always read them)
+void clear_links(tslb_ctx *c) {
+  hipLaunchKernelGGL(k_fill, dim3(grid_for(c->n)), dim3(256), 0, c->stream, (float *)c->links, 0.f, (long long)c->n);
+}
+constexpr long long kWideBytes = 0xffff0000LL;
+void set_layout(tslb_ctx *c) {
+  Params &k = c->kp;
+  const int es = (int)c->es;
+  const long long plane = (long long)k.nx * k.ny, tiles = (long long)k.tiles_x * k.tiles_y;
+  const long long lines = (tiles + line_tiles(es) - 1) / line_tiles(es);
+  const long long tiled = lines * TY * line_len(es);
+  k.tiled = 2 * tiled <= 3 * NIL * plane || tiled * k.nz <= (8LL << 20);
+  k.zsh = 0;
+  if (k.tiled) {
+    k.ps = tiled;
+  } else {
+    while ((plane << (k.zsh + 1)) <= kRowNodes) k.zsh++;
+    k.ps = (plane + kRowNodes - 1) / kRowNodes * kRowLen;
+  }
+  k.phi0 = ((k.nz - 1) / (1LL << k.zsh) + 1) * k.ps;
+  k.wide = k.ps * es > kWideBytes || k.zsh > 0;
+  c->len = (size_t)k.phi0 + c->fs;
+}
+
 int launch_zbc(tslb_ctx *c) {
   if (!c->zbc) return TSLB_OK;
   const int plane = c->prm.nx * c->prm.ny;
   with_storage(c, [&](auto tag) {
     using S = decltype(tag);
     hipLaunchKernelGGL(k_zplane_bc<S>, dim3((plane + 255) / 256), dim3(256), 0, c->stream,
-                       fields_of<S>(c->buf[c->cur], c->fs), c->w_in, c->zbc_phi ? c->phi_in : nullptr,
+                       (S *)c->buf[c->cur], c->w_in, c->zbc_phi ? c->phi_in : nullptr,
                        c->prm.ncomp, c->kp);
     return 0;
   });
@@ -2974,8 +3086,8 @@ int check_ctx(tslb_ctx *c) {
   if (rc) return rc;
   c->list_ok = 0;  // the state may change: the next curvature pass lists afresh
   if (c->prm.ncomp == 1 && c->phi_buf != c->cur) {
-    HIPCK(hipMemcpyAsync((char *)c->buf[c->cur] + TSLB_PHI * c->fs * c->es,
-                         (char *)c->buf[c->phi_buf] + TSLB_PHI * c->fs * c->es, c->n * c->es,
+    const size_t phi = (size_t)c->kp.phi0 * c->es;
+    HIPCK(hipMemcpyAsync((char *)c->buf[c->cur] + phi, (char *)c->buf[c->phi_buf] + phi, c->n * c->es,
                          hipMemcpyDeviceToDevice, c->stream));
     c->phi_buf = c->cur;
   }
@@ -3102,14 +3214,14 @@ int tslb_create(tslb_ctx **out, const tslb_params *p) {
     set_scale(k, g, sc);
   }
 
-  if (const char *v = getenv("TSLB_FUSED_VARIANT")) c->variant = atoi(v) & 7;
   int rc = TSLB_OK;
   hipError_t e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking);
   if (e != hipSuccess) {
     delete c;
     return fail(TSLB_E_HIP, std::string("hipStreamCreate failed: ") + hipGetErrorString(e));
   }
-  const size_t fb = c->fs * TSLB_NFIELDS * c->es;
+  set_layout(c);
+  const size_t fb = c->len * c->es;
   if ((rc = dev_alloc(c, (void **)&c->buf[0], fb)) || (rc = dev_alloc(c, (void **)&c->buf[1], fb)) ||
       (p->ncomp >= 2 && (rc = dev_alloc(c, (void **)&c->nrm, 4 * c->fs * sizeof(float)))) ||
       (p->ncomp >= 2 &&
@@ -3119,6 +3231,7 @@ int tslb_create(tslb_ctx **out, const tslb_params *p) {
       (p->ncomp == 2 &&
        (rc = dev_alloc(c, (void **)&c->flags_alt, 2 * (size_t)k.tiles_x * k.tiles_y * p->nz))) ||
       (p->storage == TSLB_STORAGE_FX16 && (rc = dev_alloc(c, (void **)&c->sat, 256))) ||
+      (k.wide && (rc = dev_alloc(c, (void **)&c->links, c->n * sizeof(uint32_t)))) ||
       (rc = dev_alloc(c, (void **)&c->part, (size_t)kRedBlocks * NRED * sizeof(double))) ||
       (rc = dev_alloc(c, (void **)&c->red, NRED * sizeof(double)))) {
     std::string msg = g_err;
@@ -3126,12 +3239,15 @@ int tslb_create(tslb_ctx **out, const tslb_params *p) {
     return fail(rc, msg);
   }
   // zero state: rho-1 = 0, all moments 0
-  for (int b = 0; b < 2; b++) zero_fields(c, c->buf[b], 0, TSLB_NFIELDS);
+  for (int b = 0; b < 2; b++)
+    hipLaunchKernelGGL(k_fill, dim3(grid_for(fb / 4)), dim3(256), 0, c->stream, (float *)c->buf[b], 0.f,
+                       (long long)(fb / 4));
   if (c->sat) hipLaunchKernelGGL(k_fill, dim3(1), dim3(256), 0, c->stream, (float *)c->sat, 0.f, 1);
+  if (k.wide) clear_links(c);
   k.sat = c->sat;
   if (c->nrm) {
-    const int tot = (int)(4 * c->fs);
-    hipLaunchKernelGGL(k_fill, dim3((tot + 255) / 256), dim3(256), 0, c->stream, c->nrm, 0.f, tot);
+    hipLaunchKernelGGL(k_fill, dim3(grid_for(4 * c->fs)), dim3(256), 0, c->stream, c->nrm, 0.f,
+                       (long long)(4 * c->fs));
   }
   e = hipStreamSynchronize(c->stream);
   if (e != hipSuccess) {
@@ -3177,6 +3293,7 @@ int tslb_set_isfluid(tslb_ctx *c, const int32_t *isf) {
   if (rc) return rc;
   if (!isf) {
     c->has_mask = 0;
+    if (c->kp.wide) clear_links(c);
     c->zwalls = 0;
     c->jet = 0;
     c->kp.gwall = 0;
@@ -3222,8 +3339,8 @@ int tslb_upload_field(tslb_ctx *c, int field, const float *data) {
   HIPCK(hipMemcpyAsync(tmp, data, c->n * sizeof(float), hipMemcpyHostToDevice, c->stream));
   with_storage(c, [&](auto tag) {
     using S = decltype(tag);
-    hipLaunchKernelGGL(k_to_storage<S>, dim3((unsigned)((c->n + 255) / 256)), dim3(256), 0, c->stream, tmp,
-                       field_ptr<S>(c->buf[c->cur], c->fs, field), (int)c->n, field, c->kp);
+    hipLaunchKernelGGL(k_to_storage<S>, dim3(grid_for(c->n)), dim3(256), 0, c->stream, tmp,
+                       (S *)c->buf[c->cur], 0, (int)c->n, field, c->kp);
     return 0;
   });
   HIPCK(hipGetLastError());
@@ -3248,8 +3365,8 @@ int tslb_download_field(tslb_ctx *c, int field, float *data) {
   float *tmp = (float *)c->buf[1 - c->cur];
   with_storage(c, [&](auto tag) {
     using S = decltype(tag);
-    hipLaunchKernelGGL(k_from_storage<S>, dim3((unsigned)((c->n + 255) / 256)), dim3(256), 0, c->stream,
-                       (const S *)field_ptr<S>(c->buf[c->cur], c->fs, field), tmp, (int)c->n, field, c->kp);
+    hipLaunchKernelGGL(k_from_storage<S>, dim3(grid_for(c->n)), dim3(256), 0, c->stream,
+                       (const S *)c->buf[c->cur], tmp, (int)c->n, field, c->kp);
     return 0;
   });
   HIPCK(hipGetLastError());
@@ -3306,8 +3423,16 @@ int tslb_checkpoint_write(tslb_ctx *c, const char *path, int64_t step) {
   if (ok && h.version == kCkpt16) ok = fwrite(c->kp.sc, sizeof(float), 4, fp) == 4;
   if (ok && h.version == kCkpt16) ok = fwrite(&c->kp.step, sizeof(uint32_t), 1, fp) == 1;
   for (int q = 0; ok && q < TSLB_NFIELDS; q++) {
-    hipError_t e = hipMemcpyAsync(host.data(), (char *)c->buf[c->cur] + (size_t)q * c->fs * c->es, bytes,
-                                  hipMemcpyDeviceToHost, c->stream);
+    // gathered in node order into the second buffer (scratch between steps)
+    void *tmp = c->buf[1 - c->cur];
+    with_storage(c, [&](auto tag) {
+      using S = decltype(tag);
+      hipLaunchKernelGGL(k_pack_field<S>, dim3(grid_for(c->n)), dim3(256), 0, c->stream,
+                         (const S *)c->buf[c->cur], (S *)tmp, (int)c->n, q, c->kp);
+      return 0;
+    });
+    hipError_t e = hipGetLastError();
+    if (e == hipSuccess) e = hipMemcpyAsync(host.data(), tmp, bytes, hipMemcpyDeviceToHost, c->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
     if (e != hipSuccess) {
       fclose(fp);
@@ -3372,8 +3497,17 @@ int tslb_checkpoint_read(tslb_ctx *c, const char *path, int64_t *step) {
       fclose(fp);
       return fail(TSLB_E_ARG, std::string("truncated checkpoint ") + path);
     }
-    hipError_t e = hipMemcpyAsync((char *)c->buf[c->cur] + (size_t)q * c->fs * c->es, host.data(), bytes,
-                                  hipMemcpyHostToDevice, c->stream);
+    void *tmp = c->buf[1 - c->cur];
+    hipError_t e = hipMemcpyAsync(tmp, host.data(), bytes, hipMemcpyHostToDevice, c->stream);
+    if (e == hipSuccess) {
+      with_storage(c, [&](auto tag) {
+        using S = decltype(tag);
+        hipLaunchKernelGGL(k_unpack_field<S>, dim3(grid_for(c->n)), dim3(256), 0, c->stream, (const S *)tmp,
+                           (S *)c->buf[c->cur], (int)c->n, q, c->kp);
+        return 0;
+      });
+      e = hipGetLastError();
+    }
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
     if (e != hipSuccess) {
       fclose(fp);
@@ -3404,21 +3538,19 @@ int tslb_download_normals(tslb_ctx *c, float *n3) {
 int tslb_init_equilibrium(tslb_ctx *c, int prepush) {
   int rc = check_ctx(c);
   if (rc) return rc;
-  void *base = c->buf[c->cur];
-  const int nb = (int)((c->n + 255) / 256);
-  zero_fields(c, base, TSLB_PXX, TSLB_PYZ + 1);
+  with_storage(c, [&](auto tag) {
+    using S = decltype(tag);
+    hipLaunchKernelGGL(k_zero_pi<S>, dim3(grid_for(c->n)), dim3(256), 0, c->stream, (S *)c->buf[c->cur], (int)c->n,
+                       c->kp);
+    if (c->prm.ncomp == 2 && prepush)
+      hipLaunchKernelGGL(k_prepush<S>, dim3(grid_for(c->n)), dim3(256), 0, c->stream, (const S *)c->buf[c->cur],
+                         phi_ptr<S>(c, 1 - c->cur), c->links, c->has_mask, c->kp);
+    return 0;
+  });
+  HIPCK(hipGetLastError());
   if (c->prm.ncomp == 2 && prepush) {
-    with_storage(c, [&](auto tag) {
-      using S = decltype(tag);
-      S *tmp = field_ptr<S>(c->buf[1 - c->cur], c->fs, TSLB_PHI);
-      hipLaunchKernelGGL(k_prepush<S>, dim3(nb), dim3(256), 0, c->stream, field_ptr<S>(base, c->fs, TSLB_PHI),
-                         field_ptr<S>(base, c->fs, TSLB_U), field_ptr<S>(base, c->fs, TSLB_V),
-                         field_ptr<S>(base, c->fs, TSLB_W), tmp, c->links, c->has_mask, c->kp);
-      return 0;
-    });
-    HIPCK(hipGetLastError());
-    HIPCK(hipMemcpyAsync((char *)base + TSLB_PHI * c->fs * c->es,
-                         (char *)c->buf[1 - c->cur] + TSLB_PHI * c->fs * c->es, c->n * c->es,
+    const size_t phi = (size_t)c->kp.phi0 * c->es;
+    HIPCK(hipMemcpyAsync((char *)c->buf[c->cur] + phi, (char *)c->buf[1 - c->cur] + phi, c->n * c->es,
                          hipMemcpyDeviceToDevice, c->stream));
   }
   HIPCK(hipStreamSynchronize(c->stream));
@@ -3490,9 +3622,8 @@ int tslb_upload_plane(tslb_ctx *c, int field, int k, const float *data) {
   HIPCK(hipMemcpyAsync(tmp, data, plane * sizeof(float), hipMemcpyHostToDevice, c->stream));
   with_storage(c, [&](auto tag) {
     using S = decltype(tag);
-    hipLaunchKernelGGL(k_to_storage<S>, dim3((unsigned)((plane + 255) / 256)), dim3(256), 0, c->stream, tmp,
-                       field_ptr<S>(c->buf[c->cur], c->fs, field) + plane * (size_t)k, (int)plane, field,
-                       c->kp);
+    hipLaunchKernelGGL(k_to_storage<S>, dim3(grid_for(plane)), dim3(256), 0, c->stream, tmp,
+                       (S *)c->buf[c->cur], (int)(plane * (size_t)k), (int)plane, field, c->kp);
     return 0;
   });
   HIPCK(hipGetLastError());
@@ -3541,11 +3672,11 @@ int tslb_set_storage_range(tslb_ctx *c, int field, float half_range) {
   const dim3 g((unsigned)((c->n + 255) / 256));
   for (int q = 0; q < TSLB_NFIELDS; q++) {
     if (sgrp(q) != sgrp(field)) continue;
-    fx16_t *f = field_ptr<fx16_t>(c->buf[c->cur], c->fs, q);
+    fx16_t *f = (fx16_t *)c->buf[c->cur];
     hipLaunchKernelGGL(k_from_storage<fx16_t>, g, dim3(256), 0, c->stream, (const fx16_t *)f, tmp, (int)c->n, q,
                        old);
     HIPCK(hipGetLastError());
-    hipLaunchKernelGGL(k_to_storage<fx16_t>, g, dim3(256), 0, c->stream, (const float *)tmp, f, (int)c->n, q, c->kp);
+    hipLaunchKernelGGL(k_to_storage<fx16_t>, g, dim3(256), 0, c->stream, (const float *)tmp, f, 0, (int)c->n, q, c->kp);
     HIPCK(hipGetLastError());
   }
   HIPCK(hipStreamSynchronize(c->stream));
@@ -3572,8 +3703,8 @@ int tslb_seed_noise(tslb_ctx *c, int field, float amp, int l) {
   if (field < 0 || field >= TSLB_NFIELDS) return fail(TSLB_E_ARG, "bad field");
   with_storage(c, [&](auto tag) {
     using S = decltype(tag);
-    hipLaunchKernelGGL(k_seed_noise<S>, dim3((unsigned)((c->n + 255) / 256)), dim3(256), 0, c->stream,
-                       field_ptr<S>(c->buf[c->cur], c->fs, field), field, amp, l, c->kp);
+    hipLaunchKernelGGL(k_seed_noise<S>, dim3(grid_for(c->n)), dim3(256), 0, c->stream, (S *)c->buf[c->cur], field,
+                       amp, l, c->kp);
     return 0;
   });
   HIPCK(hipGetLastError());
@@ -3590,7 +3721,7 @@ int tslb_reduce(tslb_ctx *c, double out[7]) {
   with_storage(c, [&](auto tag) {
     using S = decltype(tag);
     hipLaunchKernelGGL(k_reduce_part<S>, dim3(nblk), dim3(256), 0, c->stream,
-                       cfields_of<S>(c->buf[c->cur], c->fs), c->links, c->has_mask, c->kp, c->part);
+                       (const S *)c->buf[c->cur], c->links, c->has_mask, c->kp, c->part);
     return 0;
   });
   HIPCK(hipGetLastError());
@@ -3613,7 +3744,7 @@ int tslb_reduce_noalloc(tslb_ctx *c, double *out_dev) {
   with_storage(c, [&](auto tag) {
     using S = decltype(tag);
     hipLaunchKernelGGL(k_reduce_part<S>, dim3(nblk), dim3(256), 0, c->stream,
-                       cfields_of<S>(c->buf[c->cur], c->fs), c->links, c->has_mask, c->kp, part);
+                       (const S *)c->buf[c->cur], c->links, c->has_mask, c->kp, part);
     return 0;
   });
   HIPCK(hipGetLastError());

@@ -3039,6 +3039,30 @@ int launch_fused(tslb_ctx *c) {
 void clear_links(tslb_ctx *c) {
   hipLaunchKernelGGL(k_fill, dim3(grid_for(c->n)), dim3(256), 0, c->stream, (float *)c->links, 0.f, (long long)c->n);
 }
+// Planes of a block's z-chunk.  A block marches its chunk and two planes more
+// and spends about as long as one further plane on its start; alone on a CU it
+// takes ~0.6 of the time per plane that it takes beside a second one (64^3
+// one component: 2.0 us a plane with 64 blocks, 512x256x256: 4.4 us for two
+// blocks).  So a launch lasts
+//   (planes + 3) * (full rounds of two blocks per CU + a last round, of 0.6
+//   where one block per CU is enough for it),
+// and the chunk with the least of this is taken: 64 planes at 512^3 (32, 16
+// and the whole depth measured slower there), and on small lattices as few
+// planes as fill the chip.  At most 64: the interface lists keep one bit per
+// plane of a chunk.
+int choose_z_chunk(long long tiles, int nz, int ncu) {
+  int best = 1;
+  double least = 0;
+  for (int zc = 1; zc <= 64 && zc <= nz; zc++) {
+    const long long blocks = tiles * ((nz + zc - 1) / zc), full = blocks / (2 * ncu), rest = blocks % (2 * ncu);
+    const double cost = (zc + 3) * ((double)full + (rest == 0 ? 0.0 : (rest <= ncu ? 0.6 : 1.0)));
+    if (zc == 1 || cost <= least) {
+      least = cost;
+      best = zc;
+    }
+  }
+  return best;
+}
 constexpr long long kWideBytes = 0xffff0000LL;
 void set_layout(tslb_ctx *c) {
   Params &k = c->kp;
@@ -3171,8 +3195,6 @@ int tslb_create(tslb_ctx **out, const tslb_params *p) {
   k.tiles_x = (p->nx + TX - 1) / TX;
   k.tiles_y = (p->ny + TY - 1) / TY;
   {
-    // z-chunks of 64 planes (measured best at 512^3 among 32, 64 and the
-    // whole depth), shorter when that would leave fewer than two blocks per CU
     int ncu = 256;
     hipDeviceProp_t prop;
     if (hipGetDeviceProperties(&prop, p->device) == hipSuccess && prop.multiProcessorCount > 0)
@@ -3189,9 +3211,7 @@ int tslb_create(tslb_ctx **out, const tslb_params *p) {
     });
     if (const char *v = getenv("TSLB_CURV_BPC")) bpc = atoi(v);
     c->curv_grid = (bpc > 0 ? bpc : 6) * ncu;
-    const long long tiles = (long long)k.tiles_x * k.tiles_y;
-    int zc = 64;
-    while (zc > 8 && tiles * ((p->nz + zc - 1) / zc) < 2LL * ncu) zc /= 2;
+    int zc = choose_z_chunk((long long)k.tiles_x * k.tiles_y, p->nz, ncu);
     if (const char *v = getenv("TSLB_ZCHUNK")) zc = atoi(v);
     if (zc < 1) zc = 1;
     if (zc > 64) zc = 64;  // k_iface_list keeps one bit per plane of a chunk

@@ -36,10 +36,13 @@
 #include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
+#include <sched.h>
 #include <sys/resource.h>
 #include <sys/sysinfo.h>
 
+#include <atomic>
 #include <mutex>
+#include <thread>
 #include <type_traits>
 #include <string>
 #include <utility>
@@ -2774,6 +2777,8 @@ int scratch_setup(int dev) {
 
 constexpr int kRedBlocks = 1024;
 
+#include "host_copy.h"
+
 }  // namespace
 
 struct tslb_ctx {
@@ -2869,6 +2874,13 @@ int dev_alloc(tslb_ctx *c, void **p, size_t bytes) {
   }
   c->bytes += bytes;
   return TSLB_OK;
+}
+
+hipError_t copy_out(tslb_ctx *c, void *host, const void *dev, size_t bytes) {
+  return host_copy<true>(c->prm.device, c->stream, host, const_cast<void *>(dev), bytes);
+}
+hipError_t copy_in(tslb_ctx *c, void *dev, const void *host, size_t bytes) {
+  return host_copy<false>(c->prm.device, c->stream, const_cast<void *>(host), dev, bytes);
 }
 
 hipEvent_t take_event(tslb_ctx *c) {
@@ -3167,6 +3179,7 @@ int tslb_create(tslb_ctx **out, const tslb_params *p) {
   }
 
   tslb_ctx *c = new tslb_ctx();
+  stage_retain(p->device);
   c->prm = *p;
   c->n = (size_t)n;
   c->fs = (c->n + 63) & ~(size_t)63;
@@ -3237,6 +3250,7 @@ int tslb_create(tslb_ctx **out, const tslb_params *p) {
   int rc = TSLB_OK;
   hipError_t e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking);
   if (e != hipSuccess) {
+    stage_release(p->device);
     delete c;
     return fail(TSLB_E_HIP, std::string("hipStreamCreate failed: ") + hipGetErrorString(e));
   }
@@ -3304,6 +3318,7 @@ int tslb_destroy(tslb_ctx *c) {
   (void)hipFree(c->clo);
   (void)hipFree(c->cfeat);
   if (c->stream) (void)hipStreamDestroy(c->stream);
+  stage_release(c->prm.device);
   delete c;
   return TSLB_OK;
 }
@@ -3337,7 +3352,7 @@ int tslb_set_isfluid(tslb_ctx *c, const int32_t *isf) {
   }
   int32_t *tmp = nullptr;
   HIPCK(hipMalloc((void **)&tmp, c->n * sizeof(int32_t)));
-  hipError_t e = hipMemcpyAsync(tmp, isf, c->n * sizeof(int32_t), hipMemcpyHostToDevice, c->stream);
+  hipError_t e = copy_in(c, tmp, isf, c->n * sizeof(int32_t));
   if (e == hipSuccess) {
     hipLaunchKernelGGL(k_links, dim3((unsigned)((c->n + 255) / 256)), dim3(256), 0, c->stream, tmp,
                        c->links, c->kp);
@@ -3356,7 +3371,7 @@ int tslb_upload_field(tslb_ctx *c, int field, const float *data) {
   // stage the host floats in the second buffer (scratch between steps), then
   // convert into the state buffer (rho -> rho-1, storage type and scale)
   float *tmp = (float *)c->buf[1 - c->cur];
-  HIPCK(hipMemcpyAsync(tmp, data, c->n * sizeof(float), hipMemcpyHostToDevice, c->stream));
+  HIPCK(copy_in(c, tmp, data, c->n * sizeof(float)));
   with_storage(c, [&](auto tag) {
     using S = decltype(tag);
     hipLaunchKernelGGL(k_to_storage<S>, dim3(grid_for(c->n)), dim3(256), 0, c->stream, tmp,
@@ -3390,8 +3405,7 @@ int tslb_download_field(tslb_ctx *c, int field, float *data) {
     return 0;
   });
   HIPCK(hipGetLastError());
-  HIPCK(hipMemcpyAsync(data, tmp, c->n * sizeof(float), hipMemcpyDeviceToHost, c->stream));
-  HIPCK(hipStreamSynchronize(c->stream));
+  HIPCK(copy_out(c, data, tmp, c->n * sizeof(float)));
   return TSLB_OK;
 }
 
@@ -3452,8 +3466,7 @@ int tslb_checkpoint_write(tslb_ctx *c, const char *path, int64_t step) {
       return 0;
     });
     hipError_t e = hipGetLastError();
-    if (e == hipSuccess) e = hipMemcpyAsync(host.data(), tmp, bytes, hipMemcpyDeviceToHost, c->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+    if (e == hipSuccess) e = copy_out(c, host.data(), tmp, bytes);
     if (e != hipSuccess) {
       fclose(fp);
       return fail(TSLB_E_HIP, std::string("checkpoint copy: ") + hipGetErrorString(e));
@@ -3518,7 +3531,7 @@ int tslb_checkpoint_read(tslb_ctx *c, const char *path, int64_t *step) {
       return fail(TSLB_E_ARG, std::string("truncated checkpoint ") + path);
     }
     void *tmp = c->buf[1 - c->cur];
-    hipError_t e = hipMemcpyAsync(tmp, host.data(), bytes, hipMemcpyHostToDevice, c->stream);
+    hipError_t e = copy_in(c, tmp, host.data(), bytes);
     if (e == hipSuccess) {
       with_storage(c, [&](auto tag) {
         using S = decltype(tag);
@@ -3549,9 +3562,7 @@ int tslb_download_normals(tslb_ctx *c, float *n3) {
   // the stepping pass writes n only where it is nonzero; recompute densely
   if (c->normals_fresh != 2 && (rc = launch_normals(c, 1))) return rc;
   for (int a = 0; a < 3; a++)
-    HIPCK(hipMemcpyAsync(n3 + (size_t)a * c->n, c->nrm + (size_t)a * c->fs, c->n * sizeof(float),
-                         hipMemcpyDeviceToHost, c->stream));
-  HIPCK(hipStreamSynchronize(c->stream));
+    HIPCK(copy_out(c, n3 + (size_t)a * c->n, c->nrm + (size_t)a * c->fs, c->n * sizeof(float)));
   return TSLB_OK;
 }
 

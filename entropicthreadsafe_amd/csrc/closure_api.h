@@ -12,10 +12,12 @@ struct tslb_closure {
   size_t cap = 0, ns = 0;                // sample capacity and count
   float *feat = nullptr;                 // inputs, SoA 10 x cap
   float *aux = nullptr;                  // rho_bar, tau[6]: SoA 7 x cap
-  size_t tcap = 0;                       // training scratch: batch columns
-  int ldb = 0;
-  __bf16 *tbuf = nullptr;                // H0 | H1 | H2 | H3 | D1 | D2 | D3 | D4
+  int ncu = 0;
+  size_t icap = 0;                       // sample indices given by the caller
   int *idx = nullptr;
+  int rows = 0;                          // partial gradients and losses, one row per block
+  float *part = nullptr;
+  double *lpart = nullptr;
   double *loss = nullptr;
   float *coarse = nullptr;               // box-filter output, SoA 5 x ccap
   size_t ccap = 0;
@@ -23,8 +25,6 @@ struct tslb_closure {
 };
 
 namespace {
-
-constexpr int kTrainRows = 16 + 3 * 64 + 3 * 64 + 16;
 
 int clo_alloc(tslb_closure *m, void **p, size_t bytes) {
   hipError_t e = hipMalloc(p, bytes);
@@ -43,22 +43,6 @@ int check_model(tslb_closure *m) {
   return TSLB_OK;
 }
 
-__global__ __launch_bounds__(256) void k_sample_idx(int *__restrict__ idx, int nb, long long ns, uint32_t seed,
-                                                    uint32_t step) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= nb) return;
-  // splitmix64 of (seed, step, i)
-  uint64_t x = (uint64_t)seed * 0x9E3779B97F4A7C15ull + (uint64_t)step * 0xD1B54A32D192ED03ull + (uint64_t)i;
-  x = (x ^ (x >> 30)) * 0xBF58476D1CE4E5B9ull;
-  x = (x ^ (x >> 27)) * 0x94D049BB133111EBull;
-  x ^= x >> 31;
-  idx[i] = (int)(x % (uint64_t)ns);
-}
-__global__ __launch_bounds__(256) void k_iota(int *__restrict__ idx, int nb, int first) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i < nb) idx[i] = first + i;
-}
-
 void pack_weights(tslb_closure *m, hipStream_t st) {
   hipLaunchKernelGGL(k_mlp_pack, dim3(((kFwdBlocks + kBwdBlocks) * 64 + 255) / 256), dim3(256), 0, st, m->th,
                      m->wf, m->wb);
@@ -70,36 +54,40 @@ unsigned grid_for_tiles(long long tiles) {
   return (unsigned)(b < 1 ? 1 : b);
 }
 
-MlpTrainBufs train_bufs(tslb_closure *m) {
-  MlpTrainBufs tb;
-  __bf16 *b = m->tbuf;
-  const size_t r = (size_t)m->ldb;
-  tb.h0 = b;
-  tb.h1 = b + 16 * r;
-  tb.h2 = tb.h1 + 64 * r;
-  tb.h3 = tb.h2 + 64 * r;
-  tb.d1 = tb.h3 + 64 * r;
-  tb.d2 = tb.d1 + 64 * r;
-  tb.d3 = tb.d2 + 64 * r;
-  tb.d4 = tb.d3 + 64 * r;
-  return tb;
+// blocks (rows of partial sums) of a batch chunk
+int grad_rows(tslb_closure *m, int64_t nb) {
+  const int64_t groups = (nb + kGradTile - 1) / kGradTile;
+  return (int)(groups < m->ncu ? groups : m->ncu);
 }
 
-int ensure_train(tslb_closure *m, size_t nb) {
-  if (nb <= m->tcap) return TSLB_OK;
-  (void)hipFree(m->tbuf);
-  (void)hipFree(m->idx);
-  m->tbuf = nullptr;
-  m->idx = nullptr;
-  m->tcap = 0;
-  const size_t ldb = (nb + 31) / 32 * 32;
-  if (ldb > (size_t)INT32_MAX / kTrainRows) return fail(TSLB_E_ARG, "batch too large");
+int ensure_train(tslb_closure *m, int64_t nb, bool indices) {
   int rc;
-  if ((rc = clo_alloc(m, (void **)&m->tbuf, (size_t)kTrainRows * ldb * sizeof(__bf16))) ||
-      (rc = clo_alloc(m, (void **)&m->idx, ldb * sizeof(int))))
-    return rc;
-  m->tcap = nb;
-  m->ldb = (int)ldb;
+  if (indices && (size_t)nb > m->icap) {
+    (void)hipFree(m->idx);
+    m->idx = nullptr;
+    m->bytes -= m->icap * sizeof(int);
+    m->icap = 0;
+    if ((rc = clo_alloc(m, (void **)&m->idx, (size_t)nb * sizeof(int)))) return rc;
+    m->icap = (size_t)nb;
+  }
+  const int rows = grad_rows(m, nb);
+  if (rows > m->rows) {
+    const size_t row = kMlpNParam * sizeof(float);
+    (void)hipFree(m->part);
+    (void)hipFree(m->lpart);
+    m->part = nullptr;
+    m->lpart = nullptr;
+    m->bytes -= m->rows * (row + sizeof(double));
+    m->rows = 0;
+    if ((rc = clo_alloc(m, (void **)&m->part, rows * row))) return rc;
+    if ((rc = clo_alloc(m, (void **)&m->lpart, rows * sizeof(double)))) {
+      (void)hipFree(m->part);
+      m->part = nullptr;
+      m->bytes -= rows * row;
+      return rc;
+    }
+    m->rows = rows;
+  }
   return TSLB_OK;
 }
 
@@ -111,21 +99,21 @@ void zero_grad(tslb_closure *m) {
   hipLaunchKernelGGL(k_fill, dim3(1), dim3(256), 0, m->stream, (float *)m->loss, 0.f, 2);
 }
 
-// adds the gradient (and FP64 loss) of the samples idx[0..nb) to m->grad,
-// m->loss; ntot is the batch size the mean is taken over
-int run_grad(tslb_closure *m, int nb, int64_t ntot, float t_scale) {
-  hipStream_t st = m->stream;
+// partial gradients and FP64 losses of nb samples; ntot is the batch size the
+// mean is taken over
+void launch_grad(tslb_closure *m, const GradIdx &gi, int nb, int64_t ntot, float t_scale) {
   const float inv = (float)(1.0 / ((double)t_scale * t_scale * (double)ntot));
-  const MlpTrainBufs tb = train_bufs(m);
-  hipLaunchKernelGGL(k_mlp_fwd_bwd, dim3(grid_for_tiles((nb + 15) / 16)), dim3(256), 0, st, m->feat,
-                     (long long)m->cap, m->aux, (long long)m->cap, m->idx, nb, m->ldb, m->wf, m->wb, m->th, inv,
-                     tb, m->loss);
-  const int ksl = 512;  // columns per weight-gradient slice (multiple of 32)
-  const int nslice = (nb + ksl - 1) / ksl;
-  const int waves = kWgradJobs * nslice;
-  hipLaunchKernelGGL(k_mlp_wgrad, dim3((waves + 3) / 4), dim3(256), 0, st, tb, nb, m->ldb, ksl, m->grad);
-  HIPCK(hipGetLastError());
-  return TSLB_OK;
+  hipLaunchKernelGGL(k_mlp_grad, dim3(grad_rows(m, nb)), dim3(kGradThreads), 0, m->stream, m->feat,
+                     (long long)m->cap, m->aux, (long long)m->cap, gi, nb, m->wf, m->wb, m->th, inv, m->part,
+                     m->lpart);
+}
+// ... summed: into the parameters by one Adam step, or onto m->grad and m->loss
+template <bool ADAM>
+void launch_update(tslb_closure *m, int nb, float lr) {
+  const float b1 = 0.9f, b2 = 0.999f, t = (float)m->adam_t;
+  hipLaunchKernelGGL(k_mlp_update<ADAM>, dim3((kOffIn + 63) / 64), dim3(1024), 0, m->stream, m->part, m->lpart,
+                     grad_rows(m, nb), m->grad, m->loss, m->th, m->m1, m->m2, (__bf16 *)m->wf, (__bf16 *)m->wb, lr,
+                     b1, b2, 1e-8f, 1.f - powf(b1, t), 1.f - powf(b2, t));
 }
 
 // inputs of every node of a grid; phi (field fphi) in two-component runs only
@@ -202,6 +190,8 @@ int tslb_closure_create(tslb_closure **out, int64_t max_samples) {
     return rc;
   }
   m->cap = cap;
+  if (hipDeviceGetAttribute(&m->ncu, hipDeviceAttributeMultiprocessorCount, m->device) != hipSuccess || m->ncu < 1)
+    m->ncu = 256;
   for (float *b : {m->th, m->grad, m->m1, m->m2})
     hipLaunchKernelGGL(k_fill, dim3((kMlpNParam + 255) / 256), dim3(256), 0, m->stream, b, 0.f, kMlpNParam);
   pack_weights(m, m->stream);
@@ -215,8 +205,8 @@ int tslb_closure_destroy(tslb_closure *m) {
   (void)hipSetDevice(m->device);
   if (m->stream) (void)hipStreamSynchronize(m->stream);
   for (void *b : {(void *)m->th, (void *)m->wf, (void *)m->wb, (void *)m->grad, (void *)m->m1, (void *)m->m2,
-                  (void *)m->loss, (void *)m->feat, (void *)m->aux, (void *)m->tbuf, (void *)m->idx,
-                  (void *)m->coarse})
+                  (void *)m->loss, (void *)m->feat, (void *)m->aux, (void *)m->idx, (void *)m->part,
+                  (void *)m->lpart, (void *)m->coarse})
     (void)hipFree(b);
   if (m->stream) (void)hipStreamDestroy(m->stream);
   delete m;
@@ -358,17 +348,14 @@ int tslb_closure_loss_grad(tslb_closure *m, const int32_t *idx, int64_t nb, floa
       if (idx[i] < 0 || (size_t)idx[i] >= m->ns) return fail(TSLB_E_ARG, "sample index out of range");
   }
   const int64_t chunk = nb < kMaxChunk ? nb : kMaxChunk;
-  if ((rc = ensure_train(m, (size_t)chunk))) return rc;
+  if ((rc = ensure_train(m, chunk, idx != nullptr))) return rc;
   zero_grad(m);
   for (int64_t c0 = 0; c0 < nb; c0 += chunk) {
     const int len = (int)(nb - c0 < chunk ? nb - c0 : chunk);
-    if (idx) {
-      HIPCK(hipMemcpyAsync(m->idx, idx + c0, len * sizeof(int32_t), hipMemcpyHostToDevice, m->stream));
-    } else {
-      hipLaunchKernelGGL(k_iota, dim3((unsigned)((len + 255) / 256)), dim3(256), 0, m->stream, m->idx, len,
-                         (int)c0);
-    }
-    if ((rc = run_grad(m, len, nb, t_scale))) return rc;
+    if (idx) HIPCK(hipMemcpyAsync(m->idx, idx + c0, len * sizeof(int32_t), hipMemcpyHostToDevice, m->stream));
+    launch_grad(m, GradIdx{idx ? m->idx : nullptr, c0, 0, 0, 0, 0}, len, nb, t_scale);
+    launch_update<false>(m, len, 0.f);
+    HIPCK(hipGetLastError());
     // the next chunk's indices overwrite m->idx once this chunk is done
     if (idx) HIPCK(hipStreamSynchronize(m->stream));
   }
@@ -385,16 +372,11 @@ int tslb_closure_train(tslb_closure *m, int steps, int batch, float lr, float t_
   if (steps < 0 || batch <= 0 || batch > kMaxChunk) return fail(TSLB_E_ARG, "steps < 0 or batch outside 1..2^20");
   if (!m->ns) return fail(TSLB_E_STATE, "no samples");
   if (!(t_scale > 0.f) || !(lr > 0.f)) return fail(TSLB_E_ARG, "lr and t_scale must be positive");
-  if ((rc = ensure_train(m, (size_t)batch))) return rc;
+  if ((rc = ensure_train(m, batch, false))) return rc;
   for (int s = 0; s < steps; s++) {
-    hipLaunchKernelGGL(k_sample_idx, dim3((unsigned)((batch + 255) / 256)), dim3(256), 0, m->stream, m->idx, batch,
-                       (long long)m->ns, seed, (uint32_t)(m->adam_t + 1));
-    zero_grad(m);
-    if ((rc = run_grad(m, batch, batch, t_scale))) return rc;
     m->adam_t += 1;
-    hipLaunchKernelGGL(k_mlp_adam, dim3((kOffIn + 255) / 256), dim3(256), 0, m->stream, m->th, m->grad, m->m1, m->m2,
-                       lr, 0.9f, 0.999f, 1e-8f, m->adam_t);
-    pack_weights(m, m->stream);
+    launch_grad(m, GradIdx{nullptr, 0, (long long)m->ns, UINT64_MAX / m->ns, seed, (uint32_t)m->adam_t}, batch, batch, t_scale);
+    launch_update<true>(m, batch, lr);
   }
   HIPCK(hipGetLastError());
   if (last_loss) {

@@ -21,13 +21,11 @@
 // bias of layer 1 rides on a constant-1 input (k = 10); the other biases
 // initialise the accumulators.
 //
-// Training.  k_mlp_fwd_bwd runs forward and backward per 16-node tile with
-// the same chained layout (the backward products delta_{l-1} = W_l delta_l use
-// a second, transposed pack) and stores the BF16 activations and deltas
-// feature-major; k_mlp_wgrad contracts them over the batch on the matrix
-// cores (dW = delta H^T, K = nodes) and adds its partial sums to an FP32
-// gradient; k_mlp_adam updates the FP32 master weights.  The loss is summed in
-// FP64.
+// Training.  k_mlp_grad runs forward, backward (the backward products
+// delta_{l-1} = W_l delta_l use a second, transposed pack) and the weight
+// gradients (dW = delta H^T, K = samples) of 64 samples in one block, all
+// operands in LDS; k_mlp_update sums the blocks' FP32 gradients, updates the
+// FP32 master weights by Adam and repacks them.  The loss is summed in FP64.
 #pragma once
 
 constexpr int kMlpNF = 10, kMlpNH = 64, kMlpNO = 7;
@@ -55,9 +53,15 @@ __device__ __forceinline__ float gelu_f(float z) {
   const float e = __builtin_amdgcn_exp2f(z * fmaf(c1, z * z, c0));
   return z * __builtin_amdgcn_rcpf(1.f + e);
 }
-__device__ __forceinline__ float gelu_grad_f(float z) {
-  const float u = kGeluC * fmaf(kGeluA * z * z, z, z);
-  const float s = 1.f / (1.f + __expf(-2.f * u));
+// the sigmoid of it, refined by one Newton step to the accuracy of a division
+// (the bound on e keeps 0 * inf out of it)
+__device__ __forceinline__ float gelu_sigmoid_f(float z) {
+  constexpr float c0 = -2.f * kGeluC * 1.4426950408889634f, c1 = c0 * kGeluA;
+  const float d = 1.f + fminf(__builtin_amdgcn_exp2f(z * fmaf(c1, z * z, c0)), 1e38f);
+  const float s = __builtin_amdgcn_rcpf(d);
+  return fmaf(fmaf(-d, s, 1.f), s, s);
+}
+__device__ __forceinline__ float gelu_grad_f(float z, float s) {
   return fmaf(z * s * (1.f - s) * 2.f * kGeluC, fmaf(3.f * kGeluA, z * z, 1.f), s);
 }
 __device__ __forceinline__ float softplus_f(float x) {
@@ -103,23 +107,8 @@ __global__ __launch_bounds__(256) void k_mlp_pack(const float *__restrict__ th, 
   else bwd[(b - kFwdBlocks) * 64 + l] = v;
 }
 
-// B operand of layer 1 for node `node` (lane group g): scaled inputs 8g..8g+7,
-// the constant 1 at k = 10
-__device__ __forceinline__ bf16x8 mlp_input(const float *__restrict__ feat, long long fstride,
-                                            long long node, bool ok, int g,
-                                            const float *__restrict__ th) {
-  bf16x8 B;
-#pragma unroll
-  for (int i = 0; i < 8; i++) {
-    const int k = 8 * g + i;
-    float v = 0.f;
-    if (k < kMlpNF) v = ok ? feat[k * fstride + node] * th[kOffIn + k] : 0.f;
-    else if (k == kMlpNF) v = 1.f;
-    B[i] = (__bf16)v;
-  }
-  return B;
-}
-// the same in two halves: raw inputs of a tile loaded ahead of their use
+// B operand of layer 1 (lane group g: scaled inputs 8g..8g+7, the constant 1 at
+// k = 10) in two halves: the raw inputs of a tile are loaded ahead of their use
 struct MlpRaw {
   float v[8];
 };
@@ -232,245 +221,328 @@ __global__ __launch_bounds__(256) void k_mlp_infer(const float *__restrict__ fea
   }
 }
 
-// Training, pass 1: forward and backward of the batch samples idx[0..nb).
-// Stores, feature-major with node stride ldb (bf16): H0 (16 rows: scaled
-// inputs, the constant 1), H1..H3 (64 rows), D1..D3 (64 rows), D4 (16 rows),
-// and adds the FP64 loss sum.  inv = 1/(t_scale^2 * batch).
-struct MlpTrainBufs {
-  __bf16 *h0, *h1, *h2, *h3, *d1, *d2, *d3, *d4;
+// Training, first launch: loss and gradient of a batch, one row of partial
+// sums per block.  Column j of the batch is sample idx[j], first + j (no
+// index list), or drawn from (seed, step, j) by k_mlp_grad itself.
+//
+// A block of 16 waves takes 64 samples at a time, wave (mb, t) the 16 features
+// of block mb for the 16 samples of tile t: four activations a lane and layer
+// where one wave per tile had 16, so the chain of MFMA, GELU and exchange is
+// short and four waves per SIMD hide it.  Activations and deltas stay in LDS
+// in two forms: as the operand of the next layer's product (`ex`) and
+// feature-major (`row`), from which the block forms dW = delta H^T on the matrix
+// cores right away, K = its 64 samples, into accumulators it keeps over all its
+// groups.  inv = 1/(t_scale^2 * batch).
+//
+// Latency bounds it: a batch of 16384 is one group per CU (256 groups), and
+// takes 16 us with k_mlp_update 4.3 us.  One wave per tile, 13.6 MB of BF16
+// activations written for a second kernel that added dW with atomics, took 29 +
+// 15.5 us, and the indices, two fills, Adam and the packing a launch each, 15 us
+// more.  The weights are in LDS as they do not fit the registers: spilled, they
+// were waited for in every phase (25 us).  All 262144 samples of a fit: 86 us.
+constexpr int kGradTile = 64, kGradThreads = 1024;
+constexpr int kRowH0 = 0, kRowH1 = 16, kRowH2 = 80, kRowH3 = 144, kRowD1 = 208, kRowD2 = 272, kRowD3 = 336,
+              kRowD4 = 400, kGradRows = 416;
+// row pitch 72: the four lane groups of a store fall on different banks, and
+// 16-byte reads stay aligned
+constexpr int kGradPitch = kGradTile + 8;
+static_assert(kAux <= kMlpNF && kMlpNF < 16, "wave w brings input w and record entry w");
+
+struct GradIdx {
+  const int *idx;  // explicit columns, or null
+  long long first; // idx null, ns == 0: sample first + j
+  long long ns;    // > 0: drawn from ns samples
+  uint64_t inv;    // floor((2^64 - 1) / ns)
+  uint32_t seed, step;
 };
-__global__ __launch_bounds__(256) void k_mlp_fwd_bwd(const float *__restrict__ feat, long long fstride,
-                                                     const float *__restrict__ aux, long long astride,
-                                                     const int *__restrict__ idx, int nb, int ldb,
-                                                     const bf16x8 *__restrict__ wf, const bf16x8 *__restrict__ wb,
-                                                     const float *__restrict__ th, float inv, MlpTrainBufs tb,
-                                                     double *__restrict__ loss) {
-  const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
-  const int ntiles = (nb + 15) / 16;
-  double lsum = 0.0;
-  for (int t = blockIdx.x * 4 + (threadIdx.x >> 6); t < ntiles; t += gridDim.x * 4) {
-    const int col = t * 16 + c;  // batch column
-    const bool ok = col < nb;
-    const long long node = ok ? idx[col] : 0;
-    // ---- forward
-    const bf16x8 B1 = mlp_input(feat, fstride, node, ok, g, th);
-    if (g < 2) {  // rows 0..15: ten inputs, the constant 1, zeros
-#pragma unroll
-      for (int i = 0; i < 8; i++) tb.h0[(8 * g + i) * ldb + col] = B1[i];
-    }
-    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-    f32x4 z1[4], z2[4], z3[4];
-#pragma unroll
-    for (int mb = 0; mb < 4; mb++) z1[mb] = mfma16(wf[mb * 64 + lane], B1, zero);
-    bf16x8 B2[2], B3[2], B4[2];
-    mlp_act(z1, B2);
-    {
-      bf16x8 A[8];
-#pragma unroll
-      for (int k = 0; k < 8; k++) A[k] = wf[(4 + k) * 64 + lane];
-      mlp_hidden(A, B2, th + kOffB2, g, z2);
-    }
-    mlp_act(z2, B3);
-    {
-      bf16x8 A[8];
-#pragma unroll
-      for (int k = 0; k < 8; k++) A[k] = wf[(12 + k) * 64 + lane];
-      mlp_hidden(A, B3, th + kOffB3, g, z3);
-    }
-    mlp_act(z3, B4);
-    f32x4 o;
-    {
-      bf16x8 A[2] = {wf[20 * 64 + lane], wf[21 * 64 + lane]};
-      o = mlp_out(A, B4, th, g);
-    }
-    // activations, feature-major
-#pragma unroll
-    for (int ks = 0; ks < 2; ks++)
-#pragma unroll
-      for (int i = 0; i < 8; i++) {
-        const int f = mlp_perm(ks, g, i);
-        tb.h1[f * ldb + col] = B2[ks][i];
-        tb.h2[f * ldb + col] = B3[ks][i];
-        tb.h3[f * ldb + col] = B4[ks][i];
-      }
-    // ---- loss and output deltas (lane group 0 holds node c's outputs 0..3,
-    // group 1 outputs 4..6)
-    float o4 = __shfl(o[0], c + 16), o5 = __shfl(o[1], c + 16), o6 = __shfl(o[2], c + 16);
-    bf16x8 Bd;
-#pragma unroll
-    for (int i = 0; i < 8; i++) Bd[i] = (__bf16)0.f;
-    if (g == 0) {
-      float dlt[7] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-      if (ok) {
-        const float ov[7] = {o[0], o[1], o[2], o[3], o4, o5, o6};
-        const float s0 = th[kOffOut];
-        const float nu = s0 * softplus_f(ov[0]);
-        const float rho = aux[node];
-        float dnu = 0.f, l = 0.f;
-#pragma unroll
-        for (int k = 0; k < 6; k++) {
-          const float S = feat[k * fstride + node];
-          const float T = aux[(1 + k) * astride + node];
-          const float sk = th[kOffOut + 1 + k];
-          const float M = fmaf(-2.f * rho * nu, S, sk * ov[1 + k]);
-          const float r = M - T;
-          const float wk = k < 3 ? 1.f : 2.f;
-          l += wk * r * r;
-          const float dM = 2.f * wk * r * inv;
-          dnu += dM * (-2.f * rho * S);
-          dlt[1 + k] = dM * sk;
-        }
-        dlt[0] = dnu * s0 / (1.f + __expf(-ov[0]));
-        lsum += (double)l * (double)inv;
-      }
-#pragma unroll
-      for (int i = 0; i < 7; i++) Bd[i] = (__bf16)dlt[i];
-    }
-    if (g == 0) {  // rows 0..15: seven output deltas, zeros
-#pragma unroll
-      for (int i = 0; i < 8; i++) {
-        tb.d4[i * ldb + col] = Bd[i];
-        tb.d4[(8 + i) * ldb + col] = (__bf16)0.f;
-      }
-    }
-    // ---- backward: delta_3 = (W4 delta_4) * gelu'(z3), ...
-    f32x4 d[4];
-#pragma unroll
-    for (int mb = 0; mb < 4; mb++) {
-      const f32x4 acc = mfma16(wb[mb * 64 + lane], Bd, zero);
-#pragma unroll
-      for (int i = 0; i < 4; i++) d[mb][i] = acc[i] * gelu_grad_f(z3[mb][i]);
-    }
-    auto store_delta = [&](__bf16 *dst, bf16x8 (&Bp)[2]) {
-      // round to BF16 (the operand of the next product and of the weight gradient)
-#pragma unroll
-      for (int ks = 0; ks < 2; ks++)
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-          Bp[ks][i] = (__bf16)d[2 * ks + (i >> 2)][i & 3];
-          dst[mlp_perm(ks, g, i) * ldb + col] = Bp[ks][i];
-        }
-    };
-    bf16x8 Bp[2];
-    store_delta(tb.d3, Bp);
-#pragma unroll
-    for (int mb = 0; mb < 4; mb++) {
-      f32x4 acc = mfma16(wb[(4 + 2 * mb) * 64 + lane], Bp[0], zero);
-      acc = mfma16(wb[(4 + 2 * mb + 1) * 64 + lane], Bp[1], acc);
-#pragma unroll
-      for (int i = 0; i < 4; i++) d[mb][i] = acc[i] * gelu_grad_f(z2[mb][i]);
-    }
-    store_delta(tb.d2, Bp);
-#pragma unroll
-    for (int mb = 0; mb < 4; mb++) {
-      f32x4 acc = mfma16(wb[(12 + 2 * mb) * 64 + lane], Bp[0], zero);
-      acc = mfma16(wb[(12 + 2 * mb + 1) * 64 + lane], Bp[1], acc);
-#pragma unroll
-      for (int i = 0; i < 4; i++) d[mb][i] = acc[i] * gelu_grad_f(z1[mb][i]);
-    }
-    store_delta(tb.d1, Bp);
-  }
-  // FP64 loss: wave sum, one atomic per wave
-  for (int off = 32; off > 0; off >>= 1) lsum += __shfl_down(lsum, off);
-  if (lane == 0 && lsum != 0.0) atomicAdd(loss, lsum);
+__device__ __forceinline__ int grad_sample(const GradIdx &gi, int j) {
+  if (gi.idx) return gi.idx[j];
+  if (!gi.ns) return (int)(gi.first + j);
+  // splitmix64 of (seed, step, j)
+  uint64_t x = (uint64_t)gi.seed * 0x9E3779B97F4A7C15ull + (uint64_t)gi.step * 0xD1B54A32D192ED03ull + (uint64_t)j;
+  x = (x ^ (x >> 30)) * 0xBF58476D1CE4E5B9ull;
+  x = (x ^ (x >> 27)) * 0x94D049BB133111EBull;
+  x ^= x >> 31;
+  // x mod ns: the quotient by the reciprocal is at most two short
+  const uint64_t n = (uint64_t)gi.ns;
+  uint64_t r = x - __umul64hi(x, gi.inv) * n;
+  r -= r >= n ? n : 0;
+  r -= r >= n ? n : 0;
+  return (int)r;
 }
 
-// Training, pass 2: weight gradients on the matrix cores.  Output blocks
-// (16 x 16 of dW^T = delta H^T, or of the bias column): job j of
-// kWgradJobs, K (batch columns) split into slices of ksl columns.  The FP32
-// gradient is in the natural parameter layout; its bias entries get the
-// products with a column of ones.
-struct WgradJob {
-  int layer;  // 1..4
-  int mb;     // output-feature block (rows of delta)
-  int nb;     // input-feature block (rows of H), -1: bias
-};
-constexpr int kWgradJobs = 4 + 20 + 20 + 5;
-__device__ __forceinline__ WgradJob wgrad_job(int j) {
-  if (j < 4) return {1, j, 0};  // 16 input rows: 10 features, the bias row, zeros
-  j -= 4;
-  if (j < 20) return {2, j / 5, j % 5 == 4 ? -1 : j % 5};
-  j -= 20;
-  if (j < 20) return {3, j / 5, j % 5 == 4 ? -1 : j % 5};
-  j -= 20;
-  return {4, 0, j == 4 ? -1 : j};
-}
-__global__ __launch_bounds__(256) void k_mlp_wgrad(MlpTrainBufs tb, int nb, int ldb, int ksl,
-                                                   float *__restrict__ grad) {
-  const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
-  const int w = blockIdx.x * 4 + (threadIdx.x >> 6);
-  const int nslice = (nb + ksl - 1) / ksl;
-  if (w >= kWgradJobs * nslice) return;
-  const WgradJob jb = wgrad_job(w / nslice);
-  const int k0 = (w % nslice) * ksl, k1 = min(k0 + ksl, nb);
-  const __bf16 *D = jb.layer == 1 ? tb.d1 : (jb.layer == 2 ? tb.d2 : (jb.layer == 3 ? tb.d3 : tb.d4));
-  const __bf16 *H = jb.layer == 1 ? tb.h0 : (jb.layer == 2 ? tb.h1 : (jb.layer == 3 ? tb.h2 : tb.h3));
-  const __bf16 *drow = D + (size_t)(16 * jb.mb + c) * ldb;
-  const __bf16 *hrow = H + (size_t)(16 * (jb.nb < 0 ? 0 : jb.nb) + c) * ldb;
-  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+
+__global__ __launch_bounds__(kGradThreads) void k_mlp_grad(const float *__restrict__ feat, long long fstride,
+                                                           const float *__restrict__ aux, long long astride,
+                                                           GradIdx gi, int nb, const bf16x8 *__restrict__ wf,
+                                                           const bf16x8 *__restrict__ wb,
+                                                           const float *__restrict__ th, float inv,
+                                                           float *__restrict__ part, double *__restrict__ lpart) {
+  __shared__ alignas(16) __bf16 row[kGradRows][kGradPitch];
+  __shared__ bf16x8 ex[2][4][2][64];            // operand of the next product: [buffer][tile][K step][lane]
+  __shared__ float raw[kMlpNF + kAux][kGradTile];  // inputs and the auxiliary record
+  __shared__ bf16x8 wl[(kFwdBlocks + kBwdBlocks) * 64];  // both packs
+  __shared__ float cst[kMlpNParam - kOffB4];  // its bias, the input and output scales
+  __shared__ double lw[4];
+  const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, c = lane & 15;
+  // scalar: the matrix instructions ignore the execution mask, so a branch on
+  // the wave around them has to be a jump
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int t = w & 3, mb = w >> 2;
+  const int col = 16 * t + c;
+  for (int i = tid; i < (kFwdBlocks + kBwdBlocks) * 64; i += kGradThreads)
+    wl[i] = i < kFwdBlocks * 64 ? wf[i] : wb[i - kFwdBlocks * 64];
+  const bf16x8 *W = wl + lane, *T = W + kFwdBlocks * 64;  // block k at [k * 64]
+  const f32x4 b2 = *(const f32x4 *)(th + kOffB2 + 16 * mb + 4 * g);
+  const f32x4 b3 = *(const f32x4 *)(th + kOffB3 + 16 * mb + 4 * g);
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  if (w == 15 && lane < kMlpNParam - kOffB4) cst[lane] = th[kOffB4 + lane];
+  const float *sin = cst + (kOffIn - kOffB4), *sout = cst + (kOffOut - kOffB4);
+  __syncthreads();
+  f32x4 w2 = zero, w3 = zero, wx = zero, wy = zero;  // accumulators of dW
   bf16x8 ones;
 #pragma unroll
   for (int i = 0; i < 8; i++) ones[i] = (__bf16)(c == 0 ? 1.f : 0.f);
-  for (int k = k0; k < k1; k += 32) {
-    bf16x8 a, b;
-    if (k + 32 <= k1) {
-      // whole K step: 16-byte loads (rows start at multiples of 32 columns)
-      a = *(const bf16x8 *)(drow + k + 8 * g);
-      b = *(const bf16x8 *)(hrow + k + 8 * g);
-    } else {
+  double lsum = 0.0;
+
+  // four features of a sample: exchanged as its operand, kept feature-major
+  auto put = [&](int buf, int row0, const f32x4 &v) {
+    const bf16x4 h = __builtin_convertvector(v, bf16x4);
 #pragma unroll
-      for (int i = 0; i < 8; i++) {
-        const int col = k + 8 * g + i;
-        const bool in = col < k1;
-        a[i] = in ? drow[col] : (__bf16)0.f;
-        b[i] = in ? hrow[col] : (__bf16)0.f;
+    for (int i = 0; i < 4; i++) row[row0 + 16 * mb + 4 * g + i][col] = h[i];
+    if (buf >= 0) ((bf16x4 *)&ex[buf][t][mb >> 1][lane])[mb & 1] = h;
+  };
+  // dW block of 16 output features (rows d0..) by 16 input features (rows h0..;
+  // negative: the bias)
+  auto contract = [&](f32x4 &acc, int d0, int h0) {
+#pragma unroll
+    for (int k = 0; k < kGradTile; k += 32) {
+      const bf16x8 a = *(const bf16x8 *)&row[d0 + c][k + 8 * g];
+      const bf16x8 b = h0 < 0 ? ones : *(const bf16x8 *)&row[(h0 < 0 ? 0 : h0) + c][k + 8 * g];
+      acc = mfma16(a, b, acc);
+    }
+  };
+
+  for (int j0 = blockIdx.x * kGradTile; j0 < nb; j0 += gridDim.x * kGradTile) {
+    // ---- inputs: wave w brings input w (rows 10..15 of H0: the constant 1,
+    // zeros) and record entry w, lane = sample
+    const int j = j0 + lane;
+    const bool in = j < nb;
+    float v = 0.f, a = 0.f;
+    if (in && w < kMlpNF) {
+      const long long s = grad_sample(gi, j);
+      v = feat[w * fstride + s];
+      if (w < kAux) a = aux[w * astride + s];
+    }
+    if (w < kMlpNF) raw[w][lane] = v;
+    if (w < kAux) raw[kMlpNF + w][lane] = a;
+    row[kRowH0 + w][lane] = (__bf16)(w < kMlpNF ? (in ? v * sin[w] : 0.f) : (w == kMlpNF ? 1.f : 0.f));
+    __syncthreads();
+    // ---- forward
+    bf16x8 B;
+#pragma unroll
+    for (int i = 0; i < 8; i++) B[i] = g < 2 ? row[kRowH0 + 8 * (g & 1) + i][col] : (__bf16)0.f;
+    const f32x4 z1 = mfma16(W[mb * 64], B, zero);
+    // GELU; its derivative stays for the backward pass
+    auto act = [&](const f32x4 &z, f32x4 &dg) {
+      f32x4 h;
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const float sg = gelu_sigmoid_f(z[i]);
+        h[i] = z[i] * sg;
+        dg[i] = gelu_grad_f(z[i], sg);
       }
-    }
-    acc = mfma16(a, jb.nb < 0 ? ones : b, acc);
-  }
-  // acc[i] = sum over columns of delta[16 mb + 4g + i] * H[16 nb + c]
+      return h;
+    };
+    // the two weight blocks of a product are read ahead of the barrier before it
+    f32x4 g1, g2, g3;
+    bf16x8 A0 = W[(4 + 2 * mb) * 64], A1 = W[(5 + 2 * mb) * 64];
+    put(0, kRowH1, act(z1, g1));
+    __syncthreads();
+    f32x4 z2 = mfma16(A0, ex[0][t][0][lane], b2);
+    z2 = mfma16(A1, ex[0][t][1][lane], z2);
+    A0 = W[(12 + 2 * mb) * 64], A1 = W[(13 + 2 * mb) * 64];
+    put(1, kRowH2, act(z2, g2));
+    __syncthreads();
+    f32x4 z3 = mfma16(A0, ex[1][t][0][lane], b3);
+    z3 = mfma16(A1, ex[1][t][1][lane], z3);
+    A0 = W[20 * 64], A1 = W[21 * 64];
+    put(0, kRowH3, act(z3, g3));
+    __syncthreads();
+    // ---- loss and output deltas: one wave per tile (lane group 0 holds a
+    // sample's outputs 0..3, group 1 outputs 4..6)
+    if (mb == 0) {
+      f32x4 o;
 #pragma unroll
-  for (int i = 0; i < 4; i++) {
-    const int jo = 16 * jb.mb + 4 * g + i;  // output feature
-    const int ki = 16 * (jb.nb < 0 ? 0 : jb.nb) + c;  // input feature
-    int off = -1;
-    switch (jb.layer) {
-      case 1:
-        if (ki < kMlpNF) off = kOffW1 + ki * kMlpNH + jo;
-        else if (ki == kMlpNF) off = kOffB1 + jo;
-        break;
-      case 2:
-        if (jb.nb >= 0) off = kOffW2 + ki * kMlpNH + jo;
-        else if (c == 0) off = kOffB2 + jo;
-        break;
-      case 3:
-        if (jb.nb >= 0) off = kOffW3 + ki * kMlpNH + jo;
-        else if (c == 0) off = kOffB3 + jo;
-        break;
-      default:
-        if (jo < kMlpNO) {
-          if (jb.nb >= 0) off = kOffW4 + ki * kMlpNO + jo;
-          else if (c == 0) off = kOffB4 + jo;
+      for (int i = 0; i < 4; i++) o[i] = 4 * g + i < kMlpNO ? cst[4 * (g & 1) + i] : 0.f;
+      o = mfma16(A0, ex[0][t][0][lane], o);
+      o = mfma16(A1, ex[0][t][1][lane], o);
+      const float o4 = __shfl(o[0], c + 16), o5 = __shfl(o[1], c + 16), o6 = __shfl(o[2], c + 16);
+      bf16x8 Bd;
+#pragma unroll
+      for (int i = 0; i < 8; i++) Bd[i] = (__bf16)0.f;
+      if (g == 0) {
+        float dlt[7] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        if (j0 + col < nb) {
+          const float ov[7] = {o[0], o[1], o[2], o[3], o4, o5, o6};
+          const float s0 = sout[0];
+          const float nu = s0 * softplus_f(ov[0]);
+          const float rho = raw[kMlpNF][col];
+          float dnu = 0.f, l = 0.f;
+#pragma unroll
+          for (int k = 0; k < 6; k++) {
+            const float S = raw[k][col];
+            const float T = raw[kMlpNF + 1 + k][col];
+            const float sk = sout[1 + k];
+            const float M = fmaf(-2.f * rho * nu, S, sk * ov[1 + k]);
+            const float r = M - T;
+            const float wk = k < 3 ? 1.f : 2.f;
+            l += wk * r * r;
+            const float dM = 2.f * wk * r * inv;
+            dnu += dM * (-2.f * rho * S);
+            dlt[1 + k] = dM * sk;
+          }
+          dlt[0] = dnu * s0 / (1.f + __expf(-ov[0]));
+          lsum += (double)l * (double)inv;
         }
+#pragma unroll
+        for (int i = 0; i < 7; i++) Bd[i] = (__bf16)dlt[i];
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+          row[kRowD4 + i][col] = Bd[i];
+          row[kRowD4 + 8 + i][col] = (__bf16)0.f;
+        }
+      }
+      ex[1][t][0][lane] = Bd;
     }
-    if (off >= 0 && acc[i] != 0.f) atomicAdd(grad + off, acc[i]);
+    A0 = T[mb * 64];
+    __syncthreads();
+    // ---- backward: delta_3 = (W4 delta_4) * gelu'(z3), ...
+    put(0, kRowD3, mfma16(A0, ex[1][t][0][lane], zero) * g3);
+    A0 = T[(4 + 2 * mb) * 64], A1 = T[(5 + 2 * mb) * 64];
+    __syncthreads();
+    f32x4 acc = mfma16(A0, ex[0][t][0][lane], zero);
+    acc = mfma16(A1, ex[0][t][1][lane], acc);
+    A0 = T[(12 + 2 * mb) * 64], A1 = T[(13 + 2 * mb) * 64];
+    put(1, kRowD2, acc * g2);
+    __syncthreads();
+    acc = mfma16(A0, ex[1][t][0][lane], zero);
+    acc = mfma16(A1, ex[1][t][1][lane], acc);
+    put(-1, kRowD1, acc * g1);
+    __syncthreads();
+    // ---- dW: the 16 blocks each of layers 2 and 3, a block per wave; the four
+    // of layers 1 (its bias is input row 10) and 4 and the biases of layers 2
+    // and 3 on waves t = 0..3; the bias of layer 4 on one wave more
+    contract(w2, kRowD2 + 16 * mb, kRowH1 + 16 * t);
+    contract(w3, kRowD3 + 16 * mb, kRowH2 + 16 * t);
+    contract(wx, t == 1 ? kRowD4 : (t == 0 ? kRowD1 : (t == 2 ? kRowD2 : kRowD3)) + 16 * mb,
+             t == 0 ? kRowH0 : (t == 1 ? kRowH3 + 16 * mb : -1));
+    if (w == 0) contract(wy, kRowD4, -1);
+    __syncthreads();  // the next group overwrites the rows
+  }
+
+  // ---- partial sums in the natural parameter order: lane (g, c) of a block has
+  // outputs 16 m + 4g + i of input 16 n + c
+  float *o = part + (size_t)blockIdx.x * kMlpNParam;
+  const int m0 = 16 * mb + 4 * g;
+  *(f32x4 *)(o + kOffW2 + (16 * t + c) * kMlpNH + m0) = w2;
+  *(f32x4 *)(o + kOffW3 + (16 * t + c) * kMlpNH + m0) = w3;
+  if (t == 0) {
+    if (c < kMlpNF) *(f32x4 *)(o + kOffW1 + c * kMlpNH + m0) = wx;
+    else if (c == kMlpNF) *(f32x4 *)(o + kOffB1 + m0) = wx;
+  } else if (t == 1) {
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+      if (4 * g + i < kMlpNO) o[kOffW4 + (16 * mb + c) * kMlpNO + 4 * g + i] = wx[i];
+  } else if (c == 0) {
+    *(f32x4 *)(o + (t == 2 ? kOffB2 : kOffB3) + m0) = wx;
+  }
+  if (w == 0 && c == 0) {
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+      if (4 * g + i < kMlpNO) o[kOffB4 + 4 * g + i] = wy[i];
+  }
+  // FP64 loss: one sum per tile column, then per block
+  for (int off = 32; off > 0; off >>= 1) lsum += __shfl_down(lsum, off);
+  if (mb == 0 && lane == 0) lw[t] = lsum;
+  __syncthreads();
+  if (tid == 0) lpart[blockIdx.x] = (lw[0] + lw[1]) + (lw[2] + lw[3]);
+}
+
+// position of a weight in the packed operand blocks (the inverse of
+// k_mlp_pack): a forward and, but for layer 1 and the biases, a backward entry
+__device__ __forceinline__ void mlp_repack(int i, float x, __bf16 *__restrict__ fwd, __bf16 *__restrict__ bwd) {
+  const __bf16 h = (__bf16)x;
+  // element (row 16 mb + c, k) of a 64-wide product: block 2 mb + ks, in the order perm
+  auto hidden = [](int r, int k) {
+    const int q = k & 31;
+    return ((2 * (r >> 4) + (k >> 5)) * 64 + 16 * ((q & 15) >> 2) + (r & 15)) * 8 + 4 * (q >> 4) + (q & 3);
+  };
+  if (i < kOffW2) {  // W1 (10 x 64) and, as input 10, b1
+    const int k = i / kMlpNH, m = i % kMlpNH;
+    fwd[((m >> 4) * 64 + 16 * (k >> 3) + (m & 15)) * 8 + (k & 7)] = h;
+  } else if (i < kOffB2) {
+    const int k = (i - kOffW2) / kMlpNH, m = (i - kOffW2) % kMlpNH;
+    fwd[4 * 512 + hidden(m, k)] = h;
+    bwd[12 * 512 + hidden(k, m)] = h;
+  } else if (i >= kOffW3 && i < kOffB3) {
+    const int k = (i - kOffW3) / kMlpNH, m = (i - kOffW3) % kMlpNH;
+    fwd[12 * 512 + hidden(m, k)] = h;
+    bwd[4 * 512 + hidden(k, m)] = h;
+  } else if (i >= kOffW4 && i < kOffB4) {
+    const int k = (i - kOffW4) / kMlpNO, q = (i - kOffW4) % kMlpNO;
+    fwd[20 * 512 + hidden(q, k)] = h;
+    bwd[((k >> 4) * 64 + (k & 15)) * 8 + q] = h;
   }
 }
 
-// Adam on the weights and biases (the scales stay); t is the 1-based step
-__global__ __launch_bounds__(256) void k_mlp_adam(float *__restrict__ th, const float *__restrict__ grad,
-                                                  float *__restrict__ m1, float *__restrict__ m2, float lr,
-                                                  float b1, float b2, float eps, int t) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= kOffIn) return;
-  const float gi = grad[i];
-  const float a = fmaf(b1, m1[i], (1.f - b1) * gi);
-  const float v = fmaf(b2, m2[i], (1.f - b2) * gi * gi);
-  m1[i] = a;
-  m2[i] = v;
-  const float mh = a / (1.f - powf(b1, (float)t));
-  const float vh = v / (1.f - powf(b2, (float)t));
-  th[i] -= lr * mh / (sqrtf(vh) + eps);
+// Training, second launch: the sums of `rows` partial gradients, in a fixed
+// order, and of the partial losses.  ADAM: one Adam step (c1, c2: its bias
+// corrections) on the weights and biases (the scales stay) and their packed operands; else
+// the sums are added to grad and *loss.
+//
+// A block takes 64 parameters, its 16 waves every 16th row each: 256 rows are
+// 9.7 MB read by 149 blocks.
+template <bool ADAM>
+__global__ __launch_bounds__(1024) void k_mlp_update(const float *__restrict__ part, const double *__restrict__ lpart,
+                                                     int rows, float *__restrict__ grad, double *__restrict__ loss,
+                                                     float *__restrict__ th, float *__restrict__ m1,
+                                                     float *__restrict__ m2, __bf16 *__restrict__ fwd,
+                                                     __bf16 *__restrict__ bwd, float lr, float b1, float b2,
+                                                     float eps, float c1, float c2) {
+  __shared__ float s[16][64];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int i = blockIdx.x * 64 + lane;
+  float a = 0.f;
+  if (i < kOffIn) {
+#pragma unroll 8
+    for (int r = w; r < rows; r += 16) a += part[(size_t)r * kMlpNParam + i];
+  }
+  s[w][lane] = a;
+  __syncthreads();
+  if (blockIdx.x == 0 && w == 1) {
+    double l = 0.0;
+    for (int r = lane; r < rows; r += 64) l += lpart[r];
+    for (int off = 32; off > 0; off >>= 1) l += __shfl_down(l, off);
+    if (lane == 0) *loss = ADAM ? l : *loss + l;
+  }
+  if (w || i >= kOffIn) return;
+  float gsum = 0.f;
+#pragma unroll
+  for (int k = 0; k < 16; k++) gsum += s[k][lane];
+  if constexpr (ADAM) {
+    const float a1 = fmaf(b1, m1[i], (1.f - b1) * gsum);
+    const float v = fmaf(b2, m2[i], (1.f - b2) * gsum * gsum);
+    m1[i] = a1;
+    m2[i] = v;
+    const float mh = a1 / c1, vh = v / c2;
+    const float x = th[i] - lr * mh / (sqrtf(vh) + eps);
+    th[i] = x;
+    mlp_repack(i, x, fwd, bwd);
+  } else {
+    grad[i] += gsum;
+  }
 }
 
 // Field views for the filter and input kernels: the lattice state (storage

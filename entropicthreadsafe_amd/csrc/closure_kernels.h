@@ -53,15 +53,9 @@ __device__ __forceinline__ float gelu_f(float z) {
   const float e = __builtin_amdgcn_exp2f(z * fmaf(c1, z * z, c0));
   return z * __builtin_amdgcn_rcpf(1.f + e);
 }
-// the sigmoid of it, refined by one Newton step to the accuracy of a division
-// (the bound on e keeps 0 * inf out of it)
-__device__ __forceinline__ float gelu_sigmoid_f(float z) {
-  constexpr float c0 = -2.f * kGeluC * 1.4426950408889634f, c1 = c0 * kGeluA;
-  const float d = 1.f + fminf(__builtin_amdgcn_exp2f(z * fmaf(c1, z * z, c0)), 1e38f);
-  const float s = __builtin_amdgcn_rcpf(d);
-  return fmaf(fmaf(-d, s, 1.f), s, s);
-}
-__device__ __forceinline__ float gelu_grad_f(float z, float s) {
+__device__ __forceinline__ float gelu_grad_f(float z) {
+  const float u = kGeluC * fmaf(kGeluA * z * z, z, z);
+  const float s = 1.f / (1.f + __expf(-2.f * u));
   return fmaf(z * s * (1.f - s) * 2.f * kGeluC, fmaf(3.f * kGeluA, z * z, 1.f), s);
 }
 __device__ __forceinline__ float softplus_f(float x) {
@@ -235,11 +229,11 @@ __global__ __launch_bounds__(256) void k_mlp_infer(const float *__restrict__ fea
 // groups.  inv = 1/(t_scale^2 * batch).
 //
 // Latency bounds it: a batch of 16384 is one group per CU (256 groups), and
-// takes 16 us with k_mlp_update 4.3 us.  One wave per tile, 13.6 MB of BF16
+// takes 18 us, k_mlp_update 4.5 us.  One wave per tile, 13.6 MB of BF16
 // activations written for a second kernel that added dW with atomics, took 29 +
 // 15.5 us, and the indices, two fills, Adam and the packing a launch each, 15 us
 // more.  The weights are in LDS as they do not fit the registers: spilled, they
-// were waited for in every phase (25 us).  All 262144 samples of a fit: 86 us.
+// were waited for in every phase (25 us).
 constexpr int kGradTile = 64, kGradThreads = 1024;
 constexpr int kRowH0 = 0, kRowH1 = 16, kRowH2 = 80, kRowH3 = 144, kRowD1 = 208, kRowD2 = 272, kRowD3 = 336,
               kRowD4 = 400, kGradRows = 416;
@@ -349,9 +343,8 @@ __global__ __launch_bounds__(kGradThreads) void k_mlp_grad(const float *__restri
       f32x4 h;
 #pragma unroll
       for (int i = 0; i < 4; i++) {
-        const float sg = gelu_sigmoid_f(z[i]);
-        h[i] = z[i] * sg;
-        dg[i] = gelu_grad_f(z[i], sg);
+        h[i] = gelu_f(z[i]);
+        dg[i] = gelu_grad_f(z[i]);
       }
       return h;
     };

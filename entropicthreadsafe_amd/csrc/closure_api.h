@@ -48,10 +48,10 @@ void pack_weights(tslb_closure *m, hipStream_t st) {
                      m->wf, m->wb);
 }
 
-unsigned grid_for_tiles(long long tiles) {
-  long long b = (tiles + 3) / 4;
-  if (b > 2048) b = 2048;
-  return (unsigned)(b < 1 ? 1 : b);
+// two tiles of 16 per wave and turn, at most the four blocks that a CU holds
+unsigned infer_grid(long long n, int ncu) {
+  const long long b = (n + 127) / 128;
+  return (unsigned)(b < 4LL * ncu ? b : 4LL * ncu);
 }
 
 // blocks (rows of partial sums) of a batch chunk
@@ -117,9 +117,8 @@ void launch_update(tslb_closure *m, int nb, float lr) {
 }
 
 // inputs of every node of a grid; phi (field fphi) in two-component runs only
-template <typename View>
-void launch_features(const View &v, const Params &p, int fu, int fphi, float *feat, long long fstride, long long foff,
-                     int ncu, hipStream_t st) {
+template <typename View, typename Out>
+void launch_features(const View &v, const Params &p, int fu, int fphi, const Out &out, int ncu, hipStream_t st) {
   // z-chunks of 32 planes, shorter while there are fewer than four blocks per
   // CU (each chunk loads two planes more than it has)
   const long long tiles = (long long)((p.nx + FTX - 1) / FTX) * ((p.ny + FTY - 1) / FTY);
@@ -127,9 +126,9 @@ void launch_features(const View &v, const Params &p, int fu, int fphi, float *fe
   while (zc > 2 && tiles * ((p.nz + zc - 1) / zc) < 4LL * ncu) zc /= 2;
   const dim3 g((unsigned)(tiles * ((p.nz + zc - 1) / zc)));
   if (p.ncomp == 2)
-    hipLaunchKernelGGL((k_features<View, true>), g, dim3(FNT), 0, st, v, p, fu, fphi, feat, fstride, foff, zc);
+    hipLaunchKernelGGL((k_features<View, true, Out>), g, dim3(FNT), 0, st, v, p, fu, fphi, out, zc);
   else
-    hipLaunchKernelGGL((k_features<View, false>), g, dim3(FNT), 0, st, v, p, fu, fphi, feat, fstride, foff, zc);
+    hipLaunchKernelGGL((k_features<View, false, Out>), g, dim3(FNT), 0, st, v, p, fu, fphi, out, zc);
 }
 
 // closure fields of every node of c from its current state (before a collision)
@@ -140,10 +139,11 @@ int launch_closure(tslb_ctx *c) {
   with_storage(c, [&](auto tag) {
     using S = decltype(tag);
     StateView<S> v{(const S *)c->buf[c->cur]};
-    launch_features(v, p, TSLB_U, TSLB_PHI, c->cfeat, n, 0, c->ncu, c->stream);
+    const FeatPacked out{(bf16x8 *)c->cfeat, (bf16x2 *)(c->cfeat + 4 * n), m->th};
+    launch_features(v, p, TSLB_U, TSLB_PHI, out, c->ncu, c->stream);
     return 0;
   });
-  hipLaunchKernelGGL(k_mlp_infer, dim3(grid_for_tiles((n + 15) / 16)), dim3(256), 0, c->stream, c->cfeat, n, n,
+  hipLaunchKernelGGL(k_mlp_infer<MlpPacked>, dim3(infer_grid(n, c->ncu)), dim3(256), 0, c->stream, c->cfeat, n, n,
                      m->wf, m->th, c->clo, (long long)c->fs);
   HIPCK(hipGetLastError());
   return TSLB_OK;
@@ -152,7 +152,7 @@ int launch_closure(tslb_ctx *c) {
 int ensure_closure_fields(tslb_ctx *c) {
   int rc;
   if (!c->clo && (rc = dev_alloc(c, (void **)&c->clo, 7 * c->fs * sizeof(float)))) return rc;
-  if (!c->cfeat && (rc = dev_alloc(c, (void **)&c->cfeat, 10 * c->n * sizeof(float)))) return rc;
+  if (!c->cfeat && (rc = dev_alloc(c, (void **)&c->cfeat, 5 * c->n * sizeof(float)))) return rc;
   return TSLB_OK;
 }
 
@@ -266,7 +266,7 @@ int tslb_closure_add_samples(tslb_closure *m, tslb_ctx *c, int factor) {
     return 0;
   });
   PlainView cv{m->coarse, (long long)nc};
-  launch_features(cv, pc, 1, 4, m->feat, (long long)m->cap, (long long)m->ns, c->ncu, c->stream);
+  launch_features(cv, pc, 1, 4, FeatPlain{m->feat + m->ns, (long long)m->cap}, c->ncu, c->stream);
   HIPCK(hipGetLastError());
   HIPCK(hipStreamSynchronize(c->stream));
   m->ns += nc;
@@ -324,7 +324,7 @@ int tslb_closure_forward(tslb_closure *m, float *out) {
   if (!m->ns) return TSLB_OK;
   float *d = nullptr;
   if ((rc = clo_alloc(m, (void **)&d, kMlpNO * m->ns * sizeof(float)))) return rc;
-  hipLaunchKernelGGL(k_mlp_infer, dim3(grid_for_tiles(((long long)m->ns + 15) / 16)), dim3(256), 0, m->stream,
+  hipLaunchKernelGGL(k_mlp_infer<MlpPlain>, dim3(infer_grid((long long)m->ns, m->ncu)), dim3(256), 0, m->stream,
                      m->feat, (long long)m->cap, (long long)m->ns, m->wf, m->th, d, (long long)m->ns);
   hipError_t e = hipGetLastError();
   if (e == hipSuccess) e = hipMemcpyAsync(out, d, kMlpNO * m->ns * sizeof(float), hipMemcpyDeviceToHost, m->stream);

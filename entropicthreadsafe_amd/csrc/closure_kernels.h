@@ -102,28 +102,57 @@ __global__ __launch_bounds__(256) void k_mlp_pack(const float *__restrict__ th, 
 }
 
 // B operand of layer 1 (lane group g: scaled inputs 8g..8g+7, the constant 1 at
-// k = 10) in two halves: the raw inputs of a tile are loaded ahead of their use
-struct MlpRaw {
-  float v[8];
+// k = 10), from FP32 inputs (SoA, read ahead of their use) ...
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+struct MlpPlain {
+  struct Raw {
+    float v[8];
+  };
+  const float *f;
+  long long fstride;
+  float sc[8];
+  int g;
+  __device__ __forceinline__ MlpPlain(const float *feat, long long fs, long long, const float *th, int g_)
+      : f(feat + 8LL * g_ * fs), fstride(fs), g(g_) {
+#pragma unroll
+    for (int i = 0; i < 8; i++) sc[i] = 8 * g + i < kMlpNF ? th[kOffIn + 8 * g + i] : 0.f;
+  }
+  __device__ __forceinline__ void load(Raw &r, long long node) const {
+#pragma unroll
+    for (int i = 0; i < 8; i++) r.v[i] = 8 * g + i < kMlpNF ? f[i * fstride + node] : 0.f;
+  }
+  __device__ __forceinline__ bf16x8 operand(const Raw &r) const {
+    bf16x8 B;
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      const int k = 8 * g + i;
+      B[i] = (__bf16)(k < kMlpNF ? r.v[i] * sc[i] : (k == kMlpNF ? 1.f : 0.f));
+    }
+    return B;
+  }
 };
-__device__ __forceinline__ void mlp_load(MlpRaw &r, const float *__restrict__ feat, long long fstride,
-                                         long long node, bool ok, int g) {
+// ... or from the operand as k_features writes it: eight values a node, then two
+struct MlpPacked {
+  typedef bf16x8 Raw;
+  const bf16x8 *lo;
+  const bf16x2 *hi;
+  int g;
+  __device__ __forceinline__ MlpPacked(const float *feat, long long, long long n, const float *, int g_)
+      : lo((const bf16x8 *)feat), hi((const bf16x2 *)(feat + 4 * n)), g(g_) {}
+  __device__ __forceinline__ void load(Raw &r, long long node) const {
 #pragma unroll
-  for (int i = 0; i < 8; i++) {
-    const int k = 8 * g + i;
-    r.v[i] = (k < kMlpNF && ok) ? feat[k * fstride + node] : 0.f;
+    for (int i = 0; i < 8; i++) r[i] = (__bf16)0.f;
+    if (g == 0) {
+      r = lo[node];
+    } else if (g == 1) {
+      const bf16x2 v = hi[node];
+      r[0] = v[0];
+      r[1] = v[1];
+      r[2] = (__bf16)1.f;
+    }
   }
-}
-__device__ __forceinline__ bf16x8 mlp_scale(const MlpRaw &r, int g, const float *__restrict__ th) {
-  bf16x8 B;
-#pragma unroll
-  for (int i = 0; i < 8; i++) {
-    const int k = 8 * g + i;
-    const float v = k < kMlpNF ? r.v[i] * th[kOffIn + k] : (k == kMlpNF ? 1.f : 0.f);
-    B[i] = (__bf16)v;
-  }
-  return B;
-}
+  __device__ __forceinline__ bf16x8 operand(const Raw &r) const { return r; }
+};
 
 // GELU of four accumulator blocks, packed as the two K steps of the next layer
 __device__ __forceinline__ void mlp_act(const f32x4 (&z)[4], bf16x8 (&B)[2]) {
@@ -133,84 +162,96 @@ __device__ __forceinline__ void mlp_act(const f32x4 (&z)[4], bf16x8 (&B)[2]) {
     for (int i = 0; i < 8; i++) B[ks][i] = (__bf16)gelu_f(z[2 * ks + (i >> 2)][i & 3]);
 }
 
-// one hidden layer (64 -> 64): packed weights, block k at A[k * ST] (mb-major,
-// two K steps; ST = 1 for a register array, 64 for the LDS copy)
-template <int ST = 1>
-__device__ __forceinline__ void mlp_hidden(const bf16x8 *A, const bf16x8 (&B)[2],
-                                           const float *__restrict__ bias, int g, f32x4 (&z)[4]) {
-#pragma unroll
-  for (int mb = 0; mb < 4; mb++) {
-    f32x4 acc = *(const f32x4 *)(bias + 16 * mb + 4 * g);
-    acc = mfma16(A[(2 * mb) * ST], B[0], acc);
-    acc = mfma16(A[(2 * mb + 1) * ST], B[1], acc);
-    z[mb] = acc;
-  }
-}
-
-// output layer (64 -> 7 of 16 rows): lane group g holds outputs 4g..4g+3
-template <int ST = 1>
-__device__ __forceinline__ f32x4 mlp_out(const bf16x8 *A, const bf16x8 (&B)[2],
-                                         const float *__restrict__ th, int g) {
-  f32x4 acc;
-#pragma unroll
-  for (int i = 0; i < 4; i++) {
-    const int q = 4 * g + i;
-    acc[i] = q < kMlpNO ? th[kOffB4 + q] : 0.f;
-  }
-  acc = mfma16(A[0], B[0], acc);
-  acc = mfma16(A[ST], B[1], acc);
-  return acc;
-}
-
-// Inference: features (SoA, 10 x fstride) of n nodes -> closure fields
-// (SoA, 7 x cstride): nu_t = s0 softplus(o0), dsigma_k = s_{k+1} o_{k+1}.
-// One wave per 16-node tile.  The forward weight blocks (22.5 KiB) sit in LDS,
-// one copy per block, read as 16-byte operands per MFMA; registers stay free
-// for more waves per SIMD, which hide the MFMA -> GELU -> MFMA chain.
-__global__ __launch_bounds__(256) void k_mlp_infer(const float *__restrict__ feat, long long fstride,
-                                                   long long n, const bf16x8 *__restrict__ wf,
-                                                   const float *__restrict__ th, float *__restrict__ clo,
-                                                   long long cstride) {
+// Inference: features of n nodes (In: MlpPlain, SoA 10 x fstride, or MlpPacked)
+// -> closure fields (SoA, 7 x cstride): nu_t = s0 softplus(o0), dsigma_k =
+// s_{k+1} o_{k+1}.
+//
+// The GELU bounds it: 192 a node, each two quarter-rate instructions and five
+// others, 126 us at 128^3 for 256 CUs.  So the rest is kept small: a wave takes
+// two 16-node tiles at a time, which share the reads of the weights (in LDS, one
+// copy per block, as operands) and, the second tile's outputs taken from rows
+// 8..14 of the last product, one output pass over all 64 lanes; the inputs come
+// as finished operands.  One tile at a time, its inputs loaded and scaled by
+// predicated FP32 reads, took 205 us; this takes 159 us (262144 stored samples, read as FP32: 34 -> 26 us).
+template <typename In>
+__global__ __launch_bounds__(256, 4) void k_mlp_infer(const float *__restrict__ feat, long long fstride,
+                                                      long long n, const bf16x8 *__restrict__ wf,
+                                                      const float *__restrict__ th, float *__restrict__ clo,
+                                                      long long cstride) {
   __shared__ bf16x8 wl[kFwdBlocks * 64];
+  __shared__ alignas(16) float bl[2][kMlpNH];
   for (int i = threadIdx.x; i < kFwdBlocks * 64; i += 256) wl[i] = wf[i];
+  if (threadIdx.x < 2 * kMlpNH)
+    bl[threadIdx.x / kMlpNH][threadIdx.x % kMlpNH] =
+        th[(threadIdx.x < kMlpNH ? kOffB2 : kOffB3) + threadIdx.x % kMlpNH];
   __syncthreads();
   const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
-  const bf16x8 *A = wl + lane;  // block b at A[b * 64]
-  const long long ntiles = (n + 15) / 16;
+  const bf16x8 *A = wl + lane;       // block b at A[b * 64]
+  const bf16x8 *Ah = wl + (lane ^ 8);  // its rows 8..15 and 0..7 exchanged
+  const In in(feat, fstride, n, th, g);
+  // lane groups 0, 1 write outputs 0..3, 4..6 of the first tile, 2, 3 of the second
+  const int q0 = 4 * (g & 1);
+  float so[4], bo[4];
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    so[i] = q0 + i < kMlpNO ? th[kOffOut + q0 + i] : 0.f;
+    bo[i] = q0 + i < kMlpNO ? th[kOffB4 + q0 + i] : 0.f;
+  }
+  const long long npair = (n + 31) / 32;
   const long long nw = (long long)gridDim.x * 4;
   long long t = (long long)blockIdx.x * 4 + (threadIdx.x >> 6);
-  MlpRaw nxt;
-  mlp_load(nxt, feat, fstride, t * 16 + c, t < ntiles && t * 16 + c < n, g);
-  for (; t < ntiles; t += nw) {
-    const long long node = t * 16 + c;
-    const bool ok = node < n;
-    // keep the LDS weight reads inside the loop (hoisted, they would occupy
-    // the registers the LDS copy is meant to free)
+  auto last = [&](long long node) { return node < n ? node : n - 1; };
+  typename In::Raw nxt[2];
+  if (t < npair) {
+    in.load(nxt[0], last(t * 32 + c));
+    in.load(nxt[1], last(t * 32 + 16 + c));
+  }
+  for (; t < npair; t += nw) {
+    // keep the LDS reads inside the loop (hoisted, they would occupy the
+    // registers the LDS copy is meant to free)
     asm volatile("" ::: "memory");
-    const MlpRaw cur = nxt;  // the next tile's inputs load while this one computes
-    const long long tn = t + nw, nn = tn * 16 + c;
-    mlp_load(nxt, feat, fstride, nn, tn < ntiles && nn < n, g);
-    const bf16x8 B1 = mlp_scale(cur, g, th);
-    f32x4 z[4];
+    const bf16x8 B1[2] = {in.operand(nxt[0]), in.operand(nxt[1])};
+    if (t + nw < npair) {  // the next pair's inputs load while this one computes
+      in.load(nxt[0], last((t + nw) * 32 + c));
+      in.load(nxt[1], last((t + nw) * 32 + 16 + c));
+    }
+    f32x4 z[2][4];
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int mb = 0; mb < 4; mb++) z[mb] = mfma16(A[mb * 64], B1, zero);
-    bf16x8 B[2];
-    mlp_act(z, B);
-    mlp_hidden<64>(A + 4 * 64, B, th + kOffB2, g, z);
-    mlp_act(z, B);
-    mlp_hidden<64>(A + 12 * 64, B, th + kOffB3, g, z);
-    mlp_act(z, B);
-    const f32x4 o = mlp_out<64>(A + 20 * 64, B, th, g);
-    if (ok && g < 2) {
+    for (int mb = 0; mb < 4; mb++) {
+      const bf16x8 a = A[mb * 64];
+      z[0][mb] = mfma16(a, B1[0], zero);
+      z[1][mb] = mfma16(a, B1[1], zero);
+    }
+    bf16x8 B[2][2];
+    mlp_act(z[0], B[0]);
+    mlp_act(z[1], B[1]);
 #pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const int q = 4 * g + i;
-        if (q < kMlpNO) {
-          const float s = th[kOffOut + q];
-          clo[q * cstride + node] = q == 0 ? s * softplus_f(o[i]) : s * o[i];
-        }
+    for (int l = 0; l < 2; l++) {
+#pragma unroll
+      for (int mb = 0; mb < 4; mb++) {
+        const f32x4 b = *(const f32x4 *)&bl[l][16 * mb + 4 * g];
+        const bf16x8 a0 = A[(4 + 8 * l + 2 * mb) * 64], a1 = A[(5 + 8 * l + 2 * mb) * 64];
+#pragma unroll
+        for (int k = 0; k < 2; k++) z[k][mb] = mfma16(a1, B[k][1], mfma16(a0, B[k][0], b));
       }
+      mlp_act(z[0], B[0]);
+      mlp_act(z[1], B[1]);
+    }
+    const f32x4 b = {bo[0], bo[1], bo[2], bo[3]};
+    const f32x4 o0 = mfma16(A[21 * 64], B[0][1], mfma16(A[20 * 64], B[0][0], b));
+    const f32x4 o1 = mfma16(Ah[21 * 64], B[1][1], mfma16(Ah[20 * 64], B[1][0], b));
+    const long long node = t * 32 + 16 * (g >> 1) + c;
+    f32x4 o;
+#pragma unroll
+    for (int i = 0; i < 4; i++) o[i] = g < 2 ? o0[i] : o1[i];
+    const float sp = softplus_f(o[0]);
+    o[0] = q0 ? o[0] : sp;
+    if (node < n) {
+      float *d = clo + q0 * cstride + node;
+#pragma unroll
+      for (int i = 0; i < 3; i++) d[i * cstride] = so[i] * o[i];
+      if (q0 == 0) d[3 * cstride] = so[3] * o[3];
     }
   }
 }
@@ -630,8 +671,28 @@ __global__ __launch_bounds__(256) void k_box_filter(StateView<S> f, Params p, in
 // S from the isotropic gradient (3 sum_l w_l c_l f(x + c_l), the stencil of
 // grad_axis) of (u, v, w), grad(phi), phi; the nearest
 // interior node across a wall.  Velocity at fields fu..fu+2 and phi at field
-// fphi of a source (without PHI: phi = 0).  Output SoA 10 x fstride at
-// column offset foff.
+// fphi of a source (without PHI: phi = 0).  Out takes them as FP32 (SoA 10 x
+// stride) or as the scaled BF16 operand of the first layer.
+struct FeatPlain {
+  float *o;
+  long long stride;
+  __device__ __forceinline__ void put(long long node, const float (&v)[kMlpNF]) const {
+#pragma unroll
+    for (int k = 0; k < kMlpNF; k++) o[k * stride + node] = v[k];
+  }
+};
+struct FeatPacked {
+  bf16x8 *lo;
+  bf16x2 *hi;
+  const float *th;
+  __device__ __forceinline__ void put(long long node, const float (&v)[kMlpNF]) const {
+    bf16x8 a;
+#pragma unroll
+    for (int k = 0; k < 8; k++) a[k] = (__bf16)(v[k] * th[kOffIn + k]);
+    lo[node] = a;
+    hi[node] = bf16x2{(__bf16)(v[8] * th[kOffIn + 8]), (__bf16)(v[9] * th[kOffIn + 9])};
+  }
+};
 //
 // A 64x4 block marches a z-chunk.  It keeps four planes of its 66x6 footprint
 // in an LDS ring (25 KiB; the plane two ahead loads into registers meanwhile)
@@ -641,9 +702,8 @@ __global__ __launch_bounds__(256) void k_box_filter(StateView<S> f, Params p, in
 // written and 34 MB read: 24 us at the rate of a copy).
 constexpr int FTX = 64, FTY = 4, FSW = FTX + 2, FSH = FTY + 2, FNSLOT = FSW * FSH, FNT = FTX * FTY;
 static_assert(FNSLOT <= 2 * FNT, "at most two footprint slots per thread");
-template <typename Src, bool PHI>
-__global__ __launch_bounds__(FNT) void k_features(Src f, Params p, int fu, int fphi, float *__restrict__ feat,
-                                                  long long fstride, long long foff, int zc) {
+template <typename Src, bool PHI, typename Out>
+__global__ __launch_bounds__(FNT) void k_features(Src f, Params p, int fu, int fphi, Out out, int zc) {
   constexpr int NQ = PHI ? 4 : 3;
   __shared__ float ring[4][NQ][FNSLOT];
   const int tid = threadIdx.x, tx = tid % FTX, ty = tid / FTX;
@@ -704,16 +764,16 @@ __global__ __launch_bounds__(FNT) void k_features(Src f, Params p, int fu, int f
         if (kCZ[l]) g[q][2] = fmaf(w3 * (float)kCZ[l], v, g[q][2]);
       }
     }
-    float *o = feat + foff + ((long long)p.nx * p.ny * z + (x + p.nx * y));
-    o[0] = g[0][0];
-    o[fstride] = g[1][1];
-    o[2 * fstride] = g[2][2];
-    o[3 * fstride] = 0.5f * (g[0][1] + g[1][0]);
-    o[4 * fstride] = 0.5f * (g[0][2] + g[2][0]);
-    o[5 * fstride] = 0.5f * (g[1][2] + g[2][1]);
-    o[6 * fstride] = PHI ? g[NQ - 1][0] : 0.f;
-    o[7 * fstride] = PHI ? g[NQ - 1][1] : 0.f;
-    o[8 * fstride] = PHI ? g[NQ - 1][2] : 0.f;
-    o[9 * fstride] = PHI ? ring[(z - z0 + 4) & 3][NQ - 1][own] : 0.f;
+    const float v[kMlpNF] = {g[0][0],
+                             g[1][1],
+                             g[2][2],
+                             0.5f * (g[0][1] + g[1][0]),
+                             0.5f * (g[0][2] + g[2][0]),
+                             0.5f * (g[1][2] + g[2][1]),
+                             PHI ? g[NQ - 1][0] : 0.f,
+                             PHI ? g[NQ - 1][1] : 0.f,
+                             PHI ? g[NQ - 1][2] : 0.f,
+                             PHI ? ring[(z - z0 + 4) & 3][NQ - 1][own] : 0.f};
+    out.put((long long)p.nx * p.ny * z + (x + p.nx * y), v);
   }
 }

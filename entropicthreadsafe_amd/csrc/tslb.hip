@@ -2811,7 +2811,7 @@ struct tslb_ctx {
   // every collision by `model` from the current state
   int clo_mode = 0;
   float *clo = nullptr;    // nu_t, dsigma[6]: 7 * fs floats
-  float *cfeat = nullptr;  // closure inputs of every node: 10 * n floats
+  float *cfeat = nullptr;  // closure inputs of every node: ten BF16 values
   struct tslb_closure *model = nullptr;
   size_t bytes = 0;
   int timing = 0;

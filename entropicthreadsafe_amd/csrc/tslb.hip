@@ -1854,7 +1854,7 @@ __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(4, 8))) vo
       }
       if (tid < 2 * (z1 - z0)) flags_next[2 * ((z0 + (tid >> 1)) * tiles_plane + tile) + (tid & 1)] = 0;
       __syncthreads();
-      append_runs(ilist_wm, &ilist_base, tid, z0, z1 - z0, (int)tiles_plane, tile, ilist, ilist + 1);
+      append_runs(ilist_wm, &ilist_base, tid, z0, z1 - z0, (int)tiles_plane, tile, ilist, ilist + 2);
     }
   }
 }
@@ -2190,14 +2190,16 @@ __global__ __launch_bounds__(NTHR) void k_iface_list(const S *__restrict__ phi, 
 // gate -- the arithmetic of k_normals_tiled, so the values are the same bits.
 // Every listed tile-plane gets its kappa (zeros included) and flag byte 1,
 // so one barrier per plane suffices.  Blocks stride over the list (its
-// length read from the counter), so every wave ends its loop.  The plane
+// length read from the counter), so every wave ends its loop.  The other of the
+// two counters is cleared for the pass that lists next (a launch of its own for
+// that took 4 us and a gap, 8 % of a step on 24^3).  The plane
 // loop is unrolled over the longest run (ring slots at constant offsets) and
 // held to 80 VGPRs, which keeps three blocks per CU (51 KiB of LDS each).
 template <typename S>
 __global__ __launch_bounds__(HNT) __attribute__((amdgpu_waves_per_eu(6, 8))) void k_curv_list(const S *__restrict__ phi, float *__restrict__ kap,
                                                     uint8_t *__restrict__ flags, const int *__restrict__ cnt,
-                                                    const int *__restrict__ list, const uint32_t *__restrict__ links,
-                                                    int has_mask, Params p) {
+                                                    const int *__restrict__ list, int *__restrict__ clear,
+                                                    const uint32_t *__restrict__ links, int has_mask, Params p) {
   // rings deep enough that a slot is rewritten only two barriers after its
   // last read, so one barrier per plane orders every LDS access
   __shared__ float ph[6][HNPSLOT];
@@ -2209,6 +2211,7 @@ __global__ __launch_bounds__(HNT) __attribute__((amdgpu_waves_per_eu(6, 8))) voi
   const uint32_t pbS = (uint32_t)(plane * sizeof(S)), pb4 = (uint32_t)(plane * 4);
   const bool two = tid + HNT < HNPSLOT;
   const bool ntwo = tid + HNT < HNSLOT;
+  if (blockIdx.x == 0 && tid == 0) *clear = 0;
   const int n_entries = *cnt;
   for (int e = blockIdx.x; e < n_entries; e += gridDim.x) {
     const int ent = list[e];
@@ -2793,7 +2796,11 @@ struct tslb_ctx {
   int phi_buf = 0;  // one component: the buffer that holds phi
   float *nrm = nullptr;  // n0, n1, n2, kappa: 4 * fs floats
   uint8_t *flags = nullptr;  // per (half-tile, plane): kappa (phase field) or gradient nonzero there
-  int *ilist = nullptr;      // phase field: counter, then the runs of half-tile-planes that may carry curvature
+  // phase field: the runs of half-tile-planes that may carry curvature, their
+  // counter at ilist[lcur], the runs from ilist[lcur + 2]; the other counter is
+  // the next list's, and is zero if lclear
+  int *ilist = nullptr;
+  int lcur = 0, lclear = 0;
   uint8_t *flags_alt = nullptr;  // phase field: flags of the next step (cleared by the fused pass)
   int list_ok = 0;           // phase field: ilist describes the current state
   int ncu = 256;             // compute units of the device
@@ -2912,6 +2919,15 @@ int drain_timing(tslb_ctx *c) {
 
 int launch_closure(tslb_ctx *c);  // closure_api.h
 
+// turns to the other counter, at zero, for a pass that lists runs
+int *next_list(tslb_ctx *c) {
+  c->lcur ^= 1;
+  if (!c->lclear)
+    hipLaunchKernelGGL(k_fill, dim3(1), dim3(256), 0, c->stream, (float *)(c->ilist + c->lcur), 0.f, 1);
+  c->lclear = 0;
+  return c->ilist + c->lcur;
+}
+
 int launch_normals(tslb_ctx *c, int dense = 0) {
   hipEvent_t e0 = nullptr, e1 = nullptr;
   if (c->timing) {
@@ -2937,12 +2953,14 @@ int launch_normals(tslb_ctx *c, int dense = 0) {
       // compute those only
       const S *phi = phi_ptr<S>(c, c->cur);
       if (!c->list_ok) {  // else the last fused pass listed the runs and cleared the flags
-        hipLaunchKernelGGL(k_fill, dim3(1), dim3(256), 0, c->stream, (float *)c->ilist, 0.f, 1);
-        hipLaunchKernelGGL((k_iface_list<S>), dim3(nblk), dim3(NTHR), 0, c->stream, phi, c->flags, c->ilist,
-                           c->ilist + 1, c->kp);
+        int *list = next_list(c);
+        hipLaunchKernelGGL((k_iface_list<S>), dim3(nblk), dim3(NTHR), 0, c->stream, phi, c->flags, list, list + 2,
+                           c->kp);
       }
+      int *list = c->ilist + c->lcur;
       hipLaunchKernelGGL((k_curv_list<S>), dim3(c->curv_grid), dim3(HNT), 0, c->stream, phi, c->nrm + 3 * c->fs,
-                         c->flags, c->ilist, c->ilist + 1, c->links, c->has_mask, c->kp);
+                         c->flags, list, list + 2, c->ilist + (c->lcur ^ 1), c->links, c->has_mask, c->kp);
+      c->lclear = 1;
     }
     return 0;
   });
@@ -2968,8 +2986,7 @@ int launch_fused(tslb_ctx *c) {
   // phase field: the fused pass lists the next step's interface runs unless
   // a boundary pass still changes phi after it
   const bool build = p.ncomp == 2 && !c->jet && !c->zbc;
-  int *ilist = build ? c->ilist : nullptr;
-  if (build) hipLaunchKernelGGL(k_fill, dim3(1), dim3(256), 0, c->stream, (float *)c->ilist, 0.f, 1);
+  int *ilist = build ? next_list(c) : nullptr;
   with_storage(c, [&](auto tag) {
     using S = decltype(tag);
     const S *s = (const S *)c->buf[c->cur];
@@ -3261,7 +3278,7 @@ int tslb_create(tslb_ctx **out, const tslb_params *p) {
       (p->ncomp >= 2 &&
        (rc = dev_alloc(c, (void **)&c->flags, 2 * (size_t)k.tiles_x * k.tiles_y * p->nz))) ||
       (p->ncomp == 2 &&
-       (rc = dev_alloc(c, (void **)&c->ilist, (2 * (size_t)k.tiles_x * k.tiles_y * p->nz + 1) * sizeof(int)))) ||
+       (rc = dev_alloc(c, (void **)&c->ilist, (2 * (size_t)k.tiles_x * k.tiles_y * p->nz + 3) * sizeof(int)))) ||
       (p->ncomp == 2 &&
        (rc = dev_alloc(c, (void **)&c->flags_alt, 2 * (size_t)k.tiles_x * k.tiles_y * p->nz))) ||
       (p->storage == TSLB_STORAGE_FX16 && (rc = dev_alloc(c, (void **)&c->sat, 256))) ||

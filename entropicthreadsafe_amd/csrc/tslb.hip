@@ -2192,7 +2192,9 @@ __global__ __launch_bounds__(NTHR) void k_iface_list(const S *__restrict__ phi, 
 // so one barrier per plane suffices.  Blocks stride over the list (its
 // length read from the counter), so every wave ends its loop.  The other of the
 // two counters is cleared for the pass that lists next (a launch of its own for
-// that took 4 us and a gap, 8 % of a step on 24^3).  The plane
+// that took 4 us and a gap, 8 % of a step on 24^3).  A run of eight planes
+// takes a block 13 us, most of it latency; while the list leaves blocks of the
+// grid idle, a run's planes go to several (24^3: 13.4 -> 6 us a step).  The plane
 // loop is unrolled over the longest run (ring slots at constant offsets) and
 // held to 80 VGPRs, which keeps three blocks per CU (51 KiB of LDS each).
 template <typename S>
@@ -2213,10 +2215,15 @@ __global__ __launch_bounds__(HNT) __attribute__((amdgpu_waves_per_eu(6, 8))) voi
   const bool ntwo = tid + HNT < HNSLOT;
   if (blockIdx.x == 0 && tid == 0) *clear = 0;
   const int n_entries = *cnt;
-  for (int e = blockIdx.x; e < n_entries; e += gridDim.x) {
-    const int ent = list[e];
-    const int len = (ent & 63) + 1, half = (ent >> 6) & 1, tp0 = ent >> 7;
-    const int zs = tp0 / tiles_plane, tile = tp0 - zs * tiles_plane;
+  // short lists: a run's planes go to 2, 4 or 8 blocks
+  int split = 0;
+  while (split < 3 && (n_entries << (split + 1)) <= (int)gridDim.x) split++;
+  for (int e = blockIdx.x; e < n_entries << split; e += gridDim.x) {
+    const int ent = list[e >> split];
+    const int half = (ent >> 6) & 1, tp0 = ent >> 7, zr = tp0 / tiles_plane, tile = tp0 - zr * tiles_plane;
+    const int part = ((ent & 63) + (1 << split)) >> split, first = (e & ((1 << split) - 1)) * part;
+    const int zs = zr + first, len = min(part, (ent & 63) + 1 - first);
+    if (len <= 0) continue;
     const int x0 = (tile % p.tiles_x) * TX + half * HX, y0 = (tile / p.tiles_x) * TY;
     const int x = x0 + tx, y = y0 + ty;
     const bool active = x < p.nx && y < p.ny;

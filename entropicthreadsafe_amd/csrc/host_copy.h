@@ -8,8 +8,9 @@
 // each thread takes the next chunk, queues its transfer on the context's
 // stream and meanwhile copies its previous one.  Five fields of 512^3 to the
 // host: 265 -> 65 ms (41 GB/s), of 256^3 31 -> 10 ms, four of 301x130x187 12 ->
-// 4.4 ms.  Below 16 MB the pool costs a run's first frame what it saves (five
-// fields of 10 MB: 3.3 -> 4.0 ms the first, 3.0 -> 2.5 ms the next ones).  From the host the runtime pins the array in place, which moves
+// 4.4 ms.  Making the pool costs a run's first frame of five 10 MB fields 0.7 ms
+// (3.3 -> 4.0) and saves 0.5 ms in each of the next; a frame of four 7.6 MB fields
+// is as fast either way.  From the host the runtime pins the array in place, which moves
 // 20-28 GB/s; the slots are ahead of that only on the largest arrays (537 MB:
 // 19 -> 12 ms; 134 MB: 4.0 ms either way; 67 MB: 2.5 ms against 2.9).
 //
@@ -20,7 +21,7 @@
 // another thread's takes the runtime's path.
 #pragma once
 
-constexpr size_t kStageMinOut = 16u << 20, kStageMinIn = 256u << 20;  // bytes from which a copy is cut
+constexpr size_t kStageMinOut = 8u << 20, kStageMinIn = 256u << 20;  // bytes from which a copy is cut
 constexpr size_t kStageSlotMax = 4u << 20;
 constexpr int kStageThreads = 8;
 

@@ -13,11 +13,11 @@ struct tslb_closure {
   float *feat = nullptr;                 // inputs, SoA 10 x cap
   float *aux = nullptr;                  // rho_bar, tau[6]: SoA 7 x cap
   int ncu = 0;
-  size_t icap = 0;                       // sample indices given by the caller
+  size_t icap = 0;                       // bytes of the sample indices given by the caller
   int *idx = nullptr;
-  int rows = 0;                          // partial gradients and losses, one row per block
-  float *part = nullptr;
-  double *lpart = nullptr;
+  size_t wcap = 0;                       // bytes of the batch's columns or of one row of partial sums per block
+  void *work = nullptr;
+  double *lpart = nullptr;               // partial losses, one per block (ncu)
   double *loss = nullptr;
   float *coarse = nullptr;               // box-filter output, SoA 5 x ccap
   size_t ccap = 0;
@@ -60,34 +60,27 @@ int grad_rows(tslb_closure *m, int64_t nb) {
   return (int)(groups < m->ncu ? groups : m->ncu);
 }
 
+// largest batch whose columns are kept for k_mlp_wgrad: four slices (see there)
+constexpr int64_t kColsMax = kWgradWaves * kSlice;
+
 int ensure_train(tslb_closure *m, int64_t nb, bool indices) {
   int rc;
-  if (indices && (size_t)nb > m->icap) {
-    (void)hipFree(m->idx);
-    m->idx = nullptr;
-    m->bytes -= m->icap * sizeof(int);
-    m->icap = 0;
-    if ((rc = clo_alloc(m, (void **)&m->idx, (size_t)nb * sizeof(int)))) return rc;
-    m->icap = (size_t)nb;
-  }
-  const int rows = grad_rows(m, nb);
-  if (rows > m->rows) {
-    const size_t row = kMlpNParam * sizeof(float);
-    (void)hipFree(m->part);
-    (void)hipFree(m->lpart);
-    m->part = nullptr;
-    m->lpart = nullptr;
-    m->bytes -= m->rows * (row + sizeof(double));
-    m->rows = 0;
-    if ((rc = clo_alloc(m, (void **)&m->part, rows * row))) return rc;
-    if ((rc = clo_alloc(m, (void **)&m->lpart, rows * sizeof(double)))) {
-      (void)hipFree(m->part);
-      m->part = nullptr;
-      m->bytes -= rows * row;
-      return rc;
-    }
-    m->rows = rows;
-  }
+  auto grow = [&](void **p, size_t *cap, size_t bytes) {
+    if (bytes <= *cap) return (int)TSLB_OK;
+    (void)hipFree(*p);
+    *p = nullptr;
+    m->bytes -= *cap;
+    *cap = 0;
+    const int rc = clo_alloc(m, p, bytes);
+    if (!rc) *cap = bytes;
+    return rc;
+  };
+  if (indices && (rc = grow((void **)&m->idx, &m->icap, (size_t)nb * sizeof(int)))) return rc;
+  const size_t need = nb <= kColsMax
+                          ? (size_t)((nb + kGradTile - 1) / kGradTile) * kGradRows * kGradTile * sizeof(__bf16)
+                          : (size_t)grad_rows(m, nb) * kMlpNParam * sizeof(float);
+  if ((rc = grow(&m->work, &m->wcap, need))) return rc;
+  if (!m->lpart && (rc = clo_alloc(m, (void **)&m->lpart, (size_t)m->ncu * sizeof(double)))) return rc;
   return TSLB_OK;
 }
 
@@ -99,21 +92,29 @@ void zero_grad(tslb_closure *m) {
   hipLaunchKernelGGL(k_fill, dim3(1), dim3(256), 0, m->stream, (float *)m->loss, 0.f, 2);
 }
 
-// partial gradients and FP64 losses of nb samples; ntot is the batch size the
-// mean is taken over
-void launch_grad(tslb_closure *m, const GradIdx &gi, int nb, int64_t ntot, float t_scale) {
+// partial gradients (or the columns for k_mlp_wgrad: cols) and FP64 losses of nb
+// samples; ntot is the batch size the mean is taken over
+void launch_grad(tslb_closure *m, bool cols, const GradIdx &gi, int nb, int64_t ntot, float t_scale) {
   const float inv = (float)(1.0 / ((double)t_scale * t_scale * (double)ntot));
-  hipLaunchKernelGGL(k_mlp_grad, dim3(grad_rows(m, nb)), dim3(kGradThreads), 0, m->stream, m->feat,
-                     (long long)m->cap, m->aux, (long long)m->cap, gi, nb, m->wf, m->wb, m->th, inv, m->part,
-                     m->lpart);
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(grad_rows(m, nb)), dim3(kGradThreads), 0, m->stream, m->feat, (long long)m->cap,
+                       m->aux, (long long)m->cap, gi, nb, m->wf, m->wb, m->th, inv, (float *)m->work,
+                       (bf16x8 *)m->work, m->lpart);
+  };
+  cols ? go(k_mlp_grad<true>) : go(k_mlp_grad<false>);
 }
 // ... summed: into the parameters by one Adam step, or onto m->grad and m->loss
 template <bool ADAM>
-void launch_update(tslb_closure *m, int nb, float lr) {
-  const float b1 = 0.9f, b2 = 0.999f, t = (float)m->adam_t;
-  hipLaunchKernelGGL(k_mlp_update<ADAM>, dim3((kOffIn + 63) / 64), dim3(1024), 0, m->stream, m->part, m->lpart,
-                     grad_rows(m, nb), m->grad, m->loss, m->th, m->m1, m->m2, (__bf16 *)m->wf, (__bf16 *)m->wb, lr,
-                     b1, b2, 1e-8f, 1.f - powf(b1, t), 1.f - powf(b2, t));
+void launch_update(tslb_closure *m, bool cols, int nb, float lr) {
+  const AdamStep adam{m->th, m->m1, m->m2, (__bf16 *)m->wf, (__bf16 *)m->wb, lr, 0.9f, 0.999f, 1e-8f,
+                      (float)m->adam_t};
+  if (cols) {
+    hipLaunchKernelGGL(k_mlp_wgrad<ADAM>, dim3(kWgradJobs + 1), dim3((nb + kSlice - 1) / kSlice * 64), 0,
+                       m->stream, (const bf16x8 *)m->work, nb, m->lpart, grad_rows(m, nb), m->grad, m->loss, adam);
+  } else {
+    hipLaunchKernelGGL(k_mlp_update<ADAM>, dim3((kOffIn + 63) / 64), dim3(1024), 0, m->stream,
+                       (const float *)m->work, m->lpart, grad_rows(m, nb), m->grad, m->loss, adam);
+  }
 }
 
 // inputs of every node of a grid; phi (field fphi) in two-component runs only
@@ -205,7 +206,7 @@ int tslb_closure_destroy(tslb_closure *m) {
   (void)hipSetDevice(m->device);
   if (m->stream) (void)hipStreamSynchronize(m->stream);
   for (void *b : {(void *)m->th, (void *)m->wf, (void *)m->wb, (void *)m->grad, (void *)m->m1, (void *)m->m2,
-                  (void *)m->loss, (void *)m->feat, (void *)m->aux, (void *)m->idx, (void *)m->part,
+                  (void *)m->loss, (void *)m->feat, (void *)m->aux, (void *)m->idx, m->work,
                   (void *)m->lpart, (void *)m->coarse})
     (void)hipFree(b);
   if (m->stream) (void)hipStreamDestroy(m->stream);
@@ -350,11 +351,12 @@ int tslb_closure_loss_grad(tslb_closure *m, const int32_t *idx, int64_t nb, floa
   const int64_t chunk = nb < kMaxChunk ? nb : kMaxChunk;
   if ((rc = ensure_train(m, chunk, idx != nullptr))) return rc;
   zero_grad(m);
+  const bool cols = chunk <= kColsMax;
   for (int64_t c0 = 0; c0 < nb; c0 += chunk) {
     const int len = (int)(nb - c0 < chunk ? nb - c0 : chunk);
     if (idx) HIPCK(hipMemcpyAsync(m->idx, idx + c0, len * sizeof(int32_t), hipMemcpyHostToDevice, m->stream));
-    launch_grad(m, GradIdx{idx ? m->idx : nullptr, c0, 0, 0, 0, 0}, len, nb, t_scale);
-    launch_update<false>(m, len, 0.f);
+    launch_grad(m, cols, GradIdx{idx ? m->idx : nullptr, c0, 0, 0, 0, 0}, len, nb, t_scale);
+    launch_update<false>(m, cols, len, 0.f);
     HIPCK(hipGetLastError());
     // the next chunk's indices overwrite m->idx once this chunk is done
     if (idx) HIPCK(hipStreamSynchronize(m->stream));
@@ -373,10 +375,12 @@ int tslb_closure_train(tslb_closure *m, int steps, int batch, float lr, float t_
   if (!m->ns) return fail(TSLB_E_STATE, "no samples");
   if (!(t_scale > 0.f) || !(lr > 0.f)) return fail(TSLB_E_ARG, "lr and t_scale must be positive");
   if ((rc = ensure_train(m, batch, false))) return rc;
+  const bool cols = batch <= kColsMax;
   for (int s = 0; s < steps; s++) {
     m->adam_t += 1;
-    launch_grad(m, GradIdx{nullptr, 0, (long long)m->ns, UINT64_MAX / m->ns, seed, (uint32_t)m->adam_t}, batch, batch, t_scale);
-    launch_update<true>(m, batch, lr);
+    launch_grad(m, cols, GradIdx{nullptr, 0, (long long)m->ns, UINT64_MAX / m->ns, seed, (uint32_t)m->adam_t}, batch,
+                batch, t_scale);
+    launch_update<true>(m, cols, batch, lr);
   }
   HIPCK(hipGetLastError());
   if (last_loss) {

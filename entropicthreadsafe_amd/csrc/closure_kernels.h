@@ -25,7 +25,9 @@
 // delta_{l-1} = W_l delta_l use a second, transposed pack) and the weight
 // gradients (dW = delta H^T, K = samples) of 64 samples in one block, all
 // operands in LDS; k_mlp_update sums the blocks' FP32 gradients, updates the
-// FP32 master weights by Adam and repacks them.  The loss is summed in FP64.
+// FP32 master weights by Adam and repacks them.  Batches of up to kColsMax
+// samples keep their activations and deltas instead, and k_mlp_wgrad forms dW
+// from them in slices of 512 samples.  The loss is summed in FP64.
 #pragma once
 
 constexpr int kMlpNF = 10, kMlpNH = 64, kMlpNO = 7;
@@ -308,12 +310,16 @@ __device__ __forceinline__ int grad_sample(const GradIdx &gi, int j) {
 
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 
+// COLS: the columns of activations and deltas go to `cols`, [group of 64
+// samples][row][sample], in place of dW.
+template <bool COLS>
 __global__ __launch_bounds__(kGradThreads) void k_mlp_grad(const float *__restrict__ feat, long long fstride,
                                                            const float *__restrict__ aux, long long astride,
                                                            GradIdx gi, int nb, const bf16x8 *__restrict__ wf,
                                                            const bf16x8 *__restrict__ wb,
                                                            const float *__restrict__ th, float inv,
-                                                           float *__restrict__ part, double *__restrict__ lpart) {
+                                                           float *__restrict__ part, bf16x8 *__restrict__ cols,
+                                                           double *__restrict__ lpart) {
   __shared__ alignas(16) __bf16 row[kGradRows][kGradPitch];
   __shared__ bf16x8 ex[2][4][2][64];            // operand of the next product: [buffer][tile][K step][lane]
   __shared__ float raw[kMlpNF + kAux][kGradTile];  // inputs and the auxiliary record
@@ -465,37 +471,45 @@ __global__ __launch_bounds__(kGradThreads) void k_mlp_grad(const float *__restri
     acc = mfma16(A1, ex[1][t][1][lane], acc);
     put(-1, kRowD1, acc * g1);
     __syncthreads();
-    // ---- dW: the 16 blocks each of layers 2 and 3, a block per wave; the four
-    // of layers 1 (its bias is input row 10) and 4 and the biases of layers 2
-    // and 3 on waves t = 0..3; the bias of layer 4 on one wave more
-    contract(w2, kRowD2 + 16 * mb, kRowH1 + 16 * t);
-    contract(w3, kRowD3 + 16 * mb, kRowH2 + 16 * t);
-    contract(wx, t == 1 ? kRowD4 : (t == 0 ? kRowD1 : (t == 2 ? kRowD2 : kRowD3)) + 16 * mb,
-             t == 0 ? kRowH0 : (t == 1 ? kRowH3 + 16 * mb : -1));
-    if (w == 0) contract(wy, kRowD4, -1);
+    if constexpr (COLS) {
+      bf16x8 *o = cols + (size_t)(j0 / kGradTile) * kGradRows * (kGradTile / 8);
+      for (int i = tid; i < kGradRows * (kGradTile / 8); i += kGradThreads)
+        o[i] = *(const bf16x8 *)&row[i / (kGradTile / 8)][i % (kGradTile / 8) * 8];
+    } else {
+      // ---- dW: the 16 blocks each of layers 2 and 3, a block per wave; the four
+      // of layers 1 (its bias is input row 10) and 4 and the biases of layers 2
+      // and 3 on waves t = 0..3; the bias of layer 4 on one wave more
+      contract(w2, kRowD2 + 16 * mb, kRowH1 + 16 * t);
+      contract(w3, kRowD3 + 16 * mb, kRowH2 + 16 * t);
+      contract(wx, t == 1 ? kRowD4 : (t == 0 ? kRowD1 : (t == 2 ? kRowD2 : kRowD3)) + 16 * mb,
+               t == 0 ? kRowH0 : (t == 1 ? kRowH3 + 16 * mb : -1));
+      if (w == 0) contract(wy, kRowD4, -1);
+    }
     __syncthreads();  // the next group overwrites the rows
   }
 
-  // ---- partial sums in the natural parameter order: lane (g, c) of a block has
-  // outputs 16 m + 4g + i of input 16 n + c
-  float *o = part + (size_t)blockIdx.x * kMlpNParam;
-  const int m0 = 16 * mb + 4 * g;
-  *(f32x4 *)(o + kOffW2 + (16 * t + c) * kMlpNH + m0) = w2;
-  *(f32x4 *)(o + kOffW3 + (16 * t + c) * kMlpNH + m0) = w3;
-  if (t == 0) {
-    if (c < kMlpNF) *(f32x4 *)(o + kOffW1 + c * kMlpNH + m0) = wx;
-    else if (c == kMlpNF) *(f32x4 *)(o + kOffB1 + m0) = wx;
-  } else if (t == 1) {
+  if constexpr (!COLS) {
+    // ---- partial sums in the natural parameter order: lane (g, c) of a block has
+    // outputs 16 m + 4g + i of input 16 n + c
+    float *o = part + (size_t)blockIdx.x * kMlpNParam;
+    const int m0 = 16 * mb + 4 * g;
+    *(f32x4 *)(o + kOffW2 + (16 * t + c) * kMlpNH + m0) = w2;
+    *(f32x4 *)(o + kOffW3 + (16 * t + c) * kMlpNH + m0) = w3;
+    if (t == 0) {
+      if (c < kMlpNF) *(f32x4 *)(o + kOffW1 + c * kMlpNH + m0) = wx;
+      else if (c == kMlpNF) *(f32x4 *)(o + kOffB1 + m0) = wx;
+    } else if (t == 1) {
 #pragma unroll
-    for (int i = 0; i < 4; i++)
-      if (4 * g + i < kMlpNO) o[kOffW4 + (16 * mb + c) * kMlpNO + 4 * g + i] = wx[i];
-  } else if (c == 0) {
-    *(f32x4 *)(o + (t == 2 ? kOffB2 : kOffB3) + m0) = wx;
-  }
-  if (w == 0 && c == 0) {
+      for (int i = 0; i < 4; i++)
+        if (4 * g + i < kMlpNO) o[kOffW4 + (16 * mb + c) * kMlpNO + 4 * g + i] = wx[i];
+    } else if (c == 0) {
+      *(f32x4 *)(o + (t == 2 ? kOffB2 : kOffB3) + m0) = wx;
+    }
+    if (w == 0 && c == 0) {
 #pragma unroll
-    for (int i = 0; i < 4; i++)
-      if (4 * g + i < kMlpNO) o[kOffB4 + 4 * g + i] = wy[i];
+      for (int i = 0; i < 4; i++)
+        if (4 * g + i < kMlpNO) o[kOffB4 + 4 * g + i] = wy[i];
+    }
   }
   // FP64 loss: one sum per tile column, then per block
   for (int off = 32; off > 0; off >>= 1) lsum += __shfl_down(lsum, off);
@@ -531,23 +545,46 @@ __device__ __forceinline__ void mlp_repack(int i, float x, __bf16 *__restrict__ 
   }
 }
 
+// Adam: the 1-based step t, one parameter i with its gradient g and its state,
+// and its packed operands
+struct AdamStep {
+  float *th, *m1, *m2;
+  __bf16 *fwd, *bwd;
+  float lr, b1, b2, eps, t;
+  // 1 - b2^t cancels: the power's last bit is up to 6e-5 / t of it and scales
+  // every step, so the power is the device's, and is formed while the gradient
+  // is read
+  struct Corr {
+    float c1, c2;
+  };
+  __device__ __forceinline__ Corr corrections() const { return {1.f - powf(b1, t), 1.f - powf(b2, t)}; }
+  __device__ __forceinline__ void operator()(const Corr &k, int i, float g, float x, float a, float v) const {
+    a = fmaf(b1, a, (1.f - b1) * g);
+    v = fmaf(b2, v, (1.f - b2) * g * g);
+    m1[i] = a;
+    m2[i] = v;
+    const float mh = a / k.c1, vh = v / k.c2;
+    x -= lr * mh / (sqrtf(vh) + eps);
+    th[i] = x;
+    mlp_repack(i, x, fwd, bwd);
+  }
+};
+
 // Training, second launch: the sums of `rows` partial gradients, in a fixed
-// order, and of the partial losses.  ADAM: one Adam step (c1, c2: its bias
-// corrections) on the weights and biases (the scales stay) and their packed operands; else
-// the sums are added to grad and *loss.
+// order, and of the partial losses.  ADAM: one Adam step on the weights and
+// biases (the scales stay); else the sums are added to grad and *loss.
 //
 // A block takes 64 parameters, its 16 waves every 16th row each: 256 rows are
 // 9.7 MB read by 149 blocks.
 template <bool ADAM>
 __global__ __launch_bounds__(1024) void k_mlp_update(const float *__restrict__ part, const double *__restrict__ lpart,
                                                      int rows, float *__restrict__ grad, double *__restrict__ loss,
-                                                     float *__restrict__ th, float *__restrict__ m1,
-                                                     float *__restrict__ m2, __bf16 *__restrict__ fwd,
-                                                     __bf16 *__restrict__ bwd, float lr, float b1, float b2,
-                                                     float eps, float c1, float c2) {
+                                                     AdamStep adam) {
   __shared__ float s[16][64];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int i = blockIdx.x * 64 + lane;
+  AdamStep::Corr corr;
+  if constexpr (ADAM) corr = adam.corrections();
   float a = 0.f;
   if (i < kOffIn) {
 #pragma unroll 8
@@ -566,16 +603,123 @@ __global__ __launch_bounds__(1024) void k_mlp_update(const float *__restrict__ p
 #pragma unroll
   for (int k = 0; k < 16; k++) gsum += s[k][lane];
   if constexpr (ADAM) {
-    const float a1 = fmaf(b1, m1[i], (1.f - b1) * gsum);
-    const float v = fmaf(b2, m2[i], (1.f - b2) * gsum * gsum);
-    m1[i] = a1;
-    m2[i] = v;
-    const float mh = a1 / c1, vh = v / c2;
-    const float x = th[i] - lr * mh / (sqrtf(vh) + eps);
-    th[i] = x;
-    mlp_repack(i, x, fwd, bwd);
+    adam(corr, i, gsum, adam.th[i], adam.m1[i], adam.m2[i]);
   } else {
     grad[i] += gsum;
+  }
+}
+
+// Training, second launch after k_mlp_grad<true>: one block per dW block of 16
+// output features by 16 input features (or by the bias), one wave per slice
+// of 512 samples, each one chain of matrix instructions, added in a fixed order:
+// a partial slice first, then the others.
+//
+// The rounding of these sums decides what comes out of a training: one other
+// bit of a gradient is 1e-5 in the weights and 3e-3 in the outputs 100 steps
+// on.  Slices of 512 added with atomics gave the same sums, bit for bit with
+// one or two slices and in most runs with three or four (a partial one arrived
+// first); from five on no two runs agreed, and k_mlp_update's sums, in groups of
+// 64, lie as close to each as they to one another.  So the line is four slices.
+// Latency bounds it: one read of the columns, all of a slice in flight, 16
+// dependent MFMAs and Adam.  A step of 1024 samples takes 16.7 us, of 2048 19.0 us
+// (k_mlp_update's way 14.7 and 15.1; 31 and 32 us with atomics).
+constexpr int kSlice = 512, kWgradJobs = 4 + 20 + 20 + 5, kWgradWaves = 4;
+struct WgradJob {
+  int layer;  // 1..4
+  int mb;     // output-feature block (rows of delta)
+  int nb;     // input-feature block (rows of H), -1: bias
+};
+__device__ __forceinline__ WgradJob wgrad_job(int j) {
+  if (j < 4) return {1, j, 0};  // 16 input rows: 10 features, the bias row, zeros
+  j -= 4;
+  if (j < 20) return {2, j / 5, j % 5 == 4 ? -1 : j % 5};
+  j -= 20;
+  if (j < 20) return {3, j / 5, j % 5 == 4 ? -1 : j % 5};
+  j -= 20;
+  return {4, 0, j == 4 ? -1 : j};
+}
+// parameter of output feature jo and input feature ki (of the bias: column 0), or -1
+__device__ __forceinline__ int wgrad_param(const WgradJob &jb, int jo, int ki) {
+  switch (jb.layer) {
+    case 1:
+      return ki < kMlpNF ? kOffW1 + ki * kMlpNH + jo : (ki == kMlpNF ? kOffB1 + jo : -1);
+    case 2:
+      return jb.nb >= 0 ? kOffW2 + ki * kMlpNH + jo : (ki == 0 ? kOffB2 + jo : -1);
+    case 3:
+      return jb.nb >= 0 ? kOffW3 + ki * kMlpNH + jo : (ki == 0 ? kOffB3 + jo : -1);
+    default:
+      if (jo >= kMlpNO) return -1;
+      return jb.nb >= 0 ? kOffW4 + ki * kMlpNO + jo : (ki == 0 ? kOffB4 + jo : -1);
+  }
+}
+template <bool ADAM>
+__global__ __launch_bounds__(64 * kWgradWaves) void k_mlp_wgrad(const bf16x8 *__restrict__ cols, int nb,
+                                                                const double *__restrict__ lpart, int rows,
+                                                                float *__restrict__ grad, double *__restrict__ loss,
+                                                                AdamStep adam) {
+  __shared__ f32x4 s[kWgradWaves][64];
+  const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (blockIdx.x == kWgradJobs) {
+    if (w) return;
+    double l = 0.0;
+    for (int r = lane; r < rows; r += 64) l += lpart[r];
+    for (int off = 32; off > 0; off >>= 1) l += __shfl_down(l, off);
+    if (lane == 0) *loss = ADAM ? l : *loss + l;
+    return;
+  }
+  const WgradJob jb = wgrad_job(blockIdx.x);
+  AdamStep::Corr corr;
+  if constexpr (ADAM) corr = adam.corrections();
+  int par[4];
+  float x[4], a1[4], a2[4];
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    par[i] = wgrad_param(jb, 16 * jb.mb + 4 * g + i, 16 * (jb.nb < 0 ? 0 : jb.nb) + c);
+    if (ADAM && w == 0 && par[i] >= 0) {
+      x[i] = adam.th[par[i]];
+      a1[i] = adam.m1[par[i]];
+      a2[i] = adam.m2[par[i]];
+    }
+  }
+  constexpr int kCh = kGradTile / 8, kGroups = kSlice / kGradTile;  // 16-byte chunks of a row, groups of a slice
+  const int d0 = (jb.layer == 1 ? kRowD1 : (jb.layer == 2 ? kRowD2 : (jb.layer == 3 ? kRowD3 : kRowD4))) + 16 * jb.mb;
+  const int h0 = (jb.layer == 1 ? kRowH0 : (jb.layer == 2 ? kRowH1 : (jb.layer == 3 ? kRowH2 : kRowH3))) + 16 * jb.nb;
+  const int groups = (nb + kGradTile - 1) / kGradTile;
+  bf16x8 none, ones;
+#pragma unroll
+  for (int i = 0; i < 8; i++) {
+    none[i] = (__bf16)0.f;
+    ones[i] = (__bf16)(c == 0 ? 1.f : 0.f);
+  }
+  bf16x8 a[2 * kGroups], b[2 * kGroups];
+#pragma unroll
+  for (int k = 0; k < 2 * kGroups; k++) {
+    // groups beyond the batch: zeros
+    a[k] = none;
+    b[k] = ones;
+    const int gr = w * kGroups + k / 2;
+    if (gr < groups) {
+      const bf16x8 *p = cols + (size_t)gr * kGradRows * kCh + 4 * (k & 1) + g;
+      a[k] = p[(d0 + c) * kCh];
+      if (jb.nb >= 0) b[k] = p[(h0 + c) * kCh];
+    }
+  }
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int k = 0; k < 2 * kGroups; k++) acc = mfma16(a[k], b[k], acc);
+  s[w][lane] = acc;
+  __syncthreads();
+  if (w) return;
+  const int whole = nb / kSlice;
+  f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+  if (nb % kSlice) sum += s[whole][lane];
+  for (int k = 0; k < whole; k++) sum += s[k][lane];
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    if (par[i] < 0) continue;
+    if constexpr (ADAM) adam(corr, par[i], sum[i], x[i], a1[i], a2[i]);
+    else grad[par[i]] += sum[i];
   }
 }
 

@@ -3077,21 +3077,24 @@ void clear_links(tslb_ctx *c) {
 }
 // Planes of a block's z-chunk.  A block marches its chunk and two planes more
 // and spends about as long as one further plane on its start; alone on a CU it
-// takes ~0.6 of the time per plane that it takes beside a second one (64^3
-// one component: 2.0 us a plane with 64 blocks, 512x256x256: 4.4 us for two
-// blocks).  So a launch lasts
-//   (planes + 3) * (full rounds of two blocks per CU + a last round, of 0.6
+// takes 0.65 (most CUs idle) to 0.85 (one block on each) of the time per plane
+// that it takes beside a second one (one component, us a plane: 64^3 with 64
+// blocks 2.0; 128^3 with 256 blocks 3.1, with 512 3.7).  So a launch lasts
+//   (planes + 3) * (full rounds of two blocks per CU + a last round, of 0.75
 //   where one block per CU is enough for it),
 // and the chunk with the least of this is taken: 64 planes at 512^3 (32, 16
 // and the whole depth measured slower there), and on small lattices as few
-// planes as fill the chip.  At most 64: the interface lists keep one bit per
-// plane of a chunk.
+// planes as fill the chip.  On 40 lattices of 20^3 to 259x413x364 with three models and
+// two storage types that is the fastest measured chunk or within 0.4 % of it, as
+// with any factor of 0.72 to 0.80; 0.6 was up to 44 % off (100^3 one component
+// 44.4 us with 12 planes, 34.1 with 6; 112^3 colour 72.5 against 49.9).  At most
+// 64: the interface lists keep one bit per plane of a chunk.
 int choose_z_chunk(long long tiles, int nz, int ncu) {
   int best = 1;
   double least = 0;
   for (int zc = 1; zc <= 64 && zc <= nz; zc++) {
     const long long blocks = tiles * ((nz + zc - 1) / zc), full = blocks / (2 * ncu), rest = blocks % (2 * ncu);
-    const double cost = (zc + 3) * ((double)full + (rest == 0 ? 0.0 : (rest <= ncu ? 0.6 : 1.0)));
+    const double cost = (zc + 3) * ((double)full + (rest == 0 ? 0.0 : (rest <= ncu ? 0.75 : 1.0)));
     if (zc == 1 || cost <= least) {
       least = cost;
       best = zc;

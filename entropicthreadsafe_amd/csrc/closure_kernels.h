@@ -738,7 +738,7 @@ struct StateView {
   }
   __device__ __forceinline__ float get(int q, const Col &c, int z, const Params &p) const {
     if (q == TSLB_PHI) return ldv(base, (uint64_t)p.phi0 + (uint64_t)((long long)p.nx * p.ny * z) + c.xy, p, q);
-    return ldv(base, plane_off(p, z) + c.off + (uint32_t)(q * kRowNodes), p, q);
+    return ldv(base, plane_off(p, z) + c.off + (uint64_t)(q * p.qs), p, q);
   }
 };
 struct PlainView {

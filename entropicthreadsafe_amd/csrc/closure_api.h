@@ -88,8 +88,8 @@ int ensure_train(tslb_closure *m, int64_t nb, bool indices) {
 constexpr int64_t kMaxChunk = 1 << 20;
 
 void zero_grad(tslb_closure *m) {
-  hipLaunchKernelGGL(k_fill, dim3((kMlpNParam + 255) / 256), dim3(256), 0, m->stream, m->grad, 0.f, kMlpNParam);
-  hipLaunchKernelGGL(k_fill, dim3(1), dim3(256), 0, m->stream, (float *)m->loss, 0.f, 2);
+  fill(m->stream, m->grad, 0.f, kMlpNParam);
+  fill(m->stream, m->loss, 0.f, 2);
 }
 
 // partial gradients (or the columns for k_mlp_wgrad: cols) and FP64 losses of nb
@@ -194,7 +194,7 @@ int tslb_closure_create(tslb_closure **out, int64_t max_samples) {
   if (hipDeviceGetAttribute(&m->ncu, hipDeviceAttributeMultiprocessorCount, m->device) != hipSuccess || m->ncu < 1)
     m->ncu = 256;
   for (float *b : {m->th, m->grad, m->m1, m->m2})
-    hipLaunchKernelGGL(k_fill, dim3((kMlpNParam + 255) / 256), dim3(256), 0, m->stream, b, 0.f, kMlpNParam);
+    fill(m->stream, b, 0.f, kMlpNParam);
   pack_weights(m, m->stream);
   HIPCK(hipStreamSynchronize(m->stream));
   *out = m;
@@ -220,7 +220,7 @@ int tslb_closure_set_params(tslb_closure *m, const float *theta, int n) {
   if (!theta || n != kMlpNParam) return fail(TSLB_E_ARG, "expected TSLB_CLOSURE_NPARAM parameters");
   HIPCK(hipMemcpyAsync(m->th, theta, kMlpNParam * sizeof(float), hipMemcpyHostToDevice, m->stream));
   for (float *b : {m->m1, m->m2})
-    hipLaunchKernelGGL(k_fill, dim3((kMlpNParam + 255) / 256), dim3(256), 0, m->stream, b, 0.f, kMlpNParam);
+    fill(m->stream, b, 0.f, kMlpNParam);
   m->adam_t = 0;
   pack_weights(m, m->stream);
   HIPCK(hipStreamSynchronize(m->stream));

@@ -2666,9 +2666,13 @@ __global__ __launch_bounds__(256) void k_zero_pi(S *__restrict__ st, int n, Para
   for (int q = 0; q < 6; q++) st[o + q * p.qs] = S{};
 }
 
+#include "launch.h"
+
 __global__ __launch_bounds__(256) void k_fill(float *__restrict__ a, float v, long long n) {
-  const long long id = blockIdx.x * 256LL + threadIdx.x;
-  if (id < n) a[id] = v;
+  for (long long id = blockIdx.x * 256LL + threadIdx.x; id < n; id += gridDim.x * 256LL) a[id] = v;
+}
+void fill(hipStream_t st, void *a, float v, long long n) {
+  hipLaunchKernelGGL(k_fill, dim3(fill_blocks(n)), dim3(256), 0, st, (float *)a, v, n);
 }
 
 #include "closure_kernels.h"
@@ -2930,7 +2934,7 @@ int launch_closure(tslb_ctx *c);  // closure_api.h
 int *next_list(tslb_ctx *c) {
   c->lcur ^= 1;
   if (!c->lclear)
-    hipLaunchKernelGGL(k_fill, dim3(1), dim3(256), 0, c->stream, (float *)(c->ilist + c->lcur), 0.f, 1);
+    fill(c->stream, c->ilist + c->lcur, 0.f, 1);
   c->lclear = 0;
   return c->ilist + c->lcur;
 }
@@ -3285,15 +3289,12 @@ int tslb_create(tslb_ctx **out, const tslb_params *p) {
   }
   // zero state: rho-1 = 0, all moments 0
   for (int b = 0; b < 2; b++)
-    hipLaunchKernelGGL(k_fill, dim3(grid_for(fb / 4)), dim3(256), 0, c->stream, (float *)c->buf[b], 0.f,
-                       (long long)(fb / 4));
-  if (c->sat) hipLaunchKernelGGL(k_fill, dim3(1), dim3(256), 0, c->stream, (float *)c->sat, 0.f, 1);
+    fill(c->stream, c->buf[b], 0.f, (long long)(fb / 4));
+  if (c->sat) fill(c->stream, c->sat, 0.f, 1);
   k.sat = c->sat;
-  if (c->nrm) {
-    hipLaunchKernelGGL(k_fill, dim3(grid_for(4 * c->fs)), dim3(256), 0, c->stream, c->nrm, 0.f,
-                       (long long)(4 * c->fs));
-  }
-  e = hipStreamSynchronize(c->stream);
+  if (c->nrm) fill(c->stream, c->nrm, 0.f, (long long)(4 * c->fs));
+  e = hipGetLastError();
+  if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
   if (e != hipSuccess) {
     tslb_destroy(c);
     return fail(TSLB_E_HIP, std::string("initial fill failed: ") + hipGetErrorString(e));

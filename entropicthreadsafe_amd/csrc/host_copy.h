@@ -79,8 +79,16 @@ int stage_threads() {
 // stream
 template <bool TO_HOST>
 hipError_t host_copy(int device, hipStream_t st, void *host, void *dev, size_t bytes) {
+  auto runtime = [&] {
+    const hipError_t e = TO_HOST ? hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, st)
+                                 : hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, st);
+    return TO_HOST && e == hipSuccess ? hipStreamSynchronize(st) : e;
+  };
+  // the runtime's path may wait for long work on the stream: never with the pool
+  if (bytes < (TO_HOST ? kStageMinOut : kStageMinIn)) return runtime();
   StagePool &s = g_stage[device];
   std::unique_lock<std::mutex> lk(s.mu, std::try_to_lock);
+  if (!lk.owns_lock()) return runtime();
   const int nthr = stage_threads();
   // two chunks per thread at least, of whole 64 KiB, at most 2 MiB, or 4 MiB
   // where a large array is worth the larger pool (512^3: 65 ms a frame, 90 with
@@ -88,10 +96,9 @@ hipError_t host_copy(int device, hipStream_t st, void *host, void *dev, size_t b
   size_t chunk = (bytes / (2 * (size_t)nthr) + 0xffff) & ~(size_t)0xffff;
   const size_t most = bytes < kStageMinIn ? kStageSlotMax / 2 : kStageSlotMax;
   if (chunk > most) chunk = most;
-  if (bytes < (TO_HOST ? kStageMinOut : kStageMinIn) || !lk.owns_lock() || !stage_ready(s, chunk)) {
-    const hipError_t e = TO_HOST ? hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, st)
-                                 : hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, st);
-    return TO_HOST && e == hipSuccess ? hipStreamSynchronize(st) : e;
+  if (!stage_ready(s, chunk)) {
+    lk.unlock();
+    return runtime();
   }
   const size_t nchunk = (bytes + chunk - 1) / chunk;
   std::atomic<size_t> next{0};

@@ -794,9 +794,10 @@ struct Src {
 };
 
 // Raw buffer access.  A descriptor (gfx9 layout: 32-bit data format, no
-// stride) covers one plane of one field, so a node is a loop-invariant 32-bit
-// byte offset from a scalar base, with no per-access 64-bit address
-// arithmetic; an access past the plane reads 0 and a store there is dropped.
+// stride) covers one plane (of one plain field, or of all moments where they
+// are interleaved), so a node is a loop-invariant 32-bit byte offset from a
+// scalar base, with no per-access 64-bit address arithmetic; an access past the
+// plane reads 0 and a store there is dropped.
 constexpr int kRsrcWord3 = 0x00020000;
 typedef __amdgpu_buffer_rsrc_t rsrc_t;
 __device__ __forceinline__ rsrc_t rsrc(const void *base, uint32_t bytes) {
@@ -873,7 +874,10 @@ struct PlaneSrc {
 // lattices they cost the two-component kernels 5 spilled registers (512^3
 // emulsion 2.52 against 2.44 ms in FP32, 2.53 against 2.37 in FP16).
 constexpr uint32_t kOOB = 0x80000000u;
-constexpr uint32_t kAnyByte = 0xffffffffu;  // no bound: every offset is of a node of the lattice
+template <typename S>
+__device__ __forceinline__ rsrc_t plane_rsrc(const S *field, const Params &p) {
+  return rsrc(field, (uint32_t)p.ps * (uint32_t)sizeof(S));
+}
 template <typename S, bool PLAIN>
 __device__ __forceinline__ uint32_t lane_off(const Params &p, int x, int y) {
   if constexpr (PLAIN) return (uint32_t)(x + p.nx * y) * (uint32_t)sizeof(S);
@@ -887,9 +891,9 @@ __device__ __forceinline__ void load_node(const S *st, const Params &p, int z, u
   const S *pl = st + plane_off(p, z);
   if constexpr (PLAIN) {
 #pragma unroll
-    for (int q = 0; q < NIL; q++) v[q] = bld<S>(rsrc(pl + q * p.qs, (uint32_t)p.ps * (uint32_t)sizeof(S)), off);
+    for (int q = 0; q < NIL; q++) v[q] = bld<S>(plane_rsrc(pl + q * p.qs, p), off);
   } else {
-    const rsrc_t r = rsrc(pl, kAnyByte);
+    const rsrc_t r = plane_rsrc(pl, p);
     keep_here(off);
 #pragma unroll
     for (int q = 0; q < NIL; q++) v[q] = bld<S>(r, off + q * kRowNodes * (uint32_t)sizeof(S));
@@ -901,9 +905,9 @@ __device__ __forceinline__ void store_node(S *st, const Params &p, int z, uint32
   S *pl = st + plane_off(p, z);
   if constexpr (PLAIN) {
 #pragma unroll
-    for (int q = 0; q < NIL; q++) bst<2>(rsrc(pl + q * p.qs, (uint32_t)p.ps * (uint32_t)sizeof(S)), off, f(q));
+    for (int q = 0; q < NIL; q++) bst<2>(plane_rsrc(pl + q * p.qs, p), off, f(q));
   } else {
-    const rsrc_t r = rsrc(pl, kAnyByte);
+    const rsrc_t r = plane_rsrc(pl, p);
     keep_here(off);
 #pragma unroll
     for (int q = 0; q < NIL; q++) bst<2>(r, off + q * kRowNodes * (uint32_t)sizeof(S), f(q));

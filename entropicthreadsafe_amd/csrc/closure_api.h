@@ -29,6 +29,7 @@ namespace {
 int clo_alloc(tslb_closure *m, void **p, size_t bytes) {
   hipError_t e = hipMalloc(p, bytes);
   if (e != hipSuccess) {
+    (void)hipGetLastError();
     *p = nullptr;
     return fail(TSLB_E_NOMEM, "hipMalloc of " + std::to_string(bytes) + " bytes failed: " +
                                   hipGetErrorString(e));

@@ -2890,6 +2890,7 @@ unsigned grid_for(size_t n) { return (unsigned)((n + 255) / 256); }
 int dev_alloc(tslb_ctx *c, void **p, size_t bytes) {
   hipError_t e = hipMalloc(p, bytes);
   if (e != hipSuccess) {
+    (void)hipGetLastError();  // reported here, not by the next launch
     *p = nullptr;
     return fail(TSLB_E_NOMEM, "hipMalloc of " + std::to_string(bytes) + " bytes failed: " +
                                   hipGetErrorString(e));
@@ -3095,7 +3096,7 @@ int choose_z_chunk(long long tiles, int nz, int ncu) {
 // where a plane fills rows (2C FP32 a step: 65x9x3000 165 -> 141 us, 16x16x8192
 // 176 -> 168).
 constexpr long long kPlaneBytes = 0xffff0000LL;  // largest plane of rows
-void set_layout(tslb_ctx *c) {
+void set_layout(tslb_ctx *c, bool padded) {
   Params &k = c->kp;
   const int es = (int)c->es;
   const long long plane = (long long)k.nx * k.ny, nt = (long long)k.tiles_x * k.tiles_y;
@@ -3104,7 +3105,7 @@ void set_layout(tslb_ctx *c) {
   const bool tiles = 2 * tiled <= 3 * NIL * plane || tiled * k.nz <= (8LL << 20);
   k.ps = tiles ? tiled : (plane + kRowNodes - 1) / kRowNodes * kRowLen;
   k.layout = tiles ? LAY_TILES : (2 * plane <= kRowNodes ? LAY_PLAIN : LAY_ROWS);
-  if (k.ps * es > kPlaneBytes) k.layout = LAY_PLAIN;
+  if (!padded || k.ps * es > kPlaneBytes) k.layout = LAY_PLAIN;
   k.qs = kRowNodes;
   k.phi0 = k.nz * k.ps;
   if (k.layout == LAY_PLAIN) {
@@ -3113,6 +3114,19 @@ void set_layout(tslb_ctx *c) {
     k.phi0 = NIL * k.qs;
   }
   c->len = (size_t)k.phi0 + c->fs;
+}
+
+// Plain fields need the least memory.  They are taken where the padding of the
+// layout's rows would leave too little of what is free for the context itself,
+// for a mask (8 bytes a node while it is set) or for a closure (48 more) that plain
+// fields leave room for; 256 MiB of slack cover the allocations' own rounding.
+bool padding_fits(const tslb_ctx *c, size_t fixed) {
+  size_t avail = 0, total = 0;
+  if (hipMemGetInfo(&avail, &total) != hipSuccess) return (void)hipGetLastError(), true;
+  const size_t padded = 2 * c->len * c->es + fixed, plain = 2 * (NIL + 1) * c->fs * c->es + fixed;
+  for (const size_t later : {0 * c->n, 8 * c->n, 56 * c->n})
+    if (plain + later <= avail && padded + later + (256u << 20) > avail) return false;
+  return true;
 }
 
 int launch_zbc(tslb_ctx *c) {
@@ -3274,16 +3288,18 @@ int tslb_create(tslb_ctx **out, const tslb_params *p) {
     delete c;
     return fail(TSLB_E_HIP, std::string("hipStreamCreate failed: ") + hipGetErrorString(e));
   }
-  set_layout(c);
+  const size_t half_tiles = 2 * (size_t)k.tiles_x * k.tiles_y * p->nz;
+  const size_t nrm_bytes = p->ncomp >= 2 ? 4 * c->fs * sizeof(float) : 0;
+  const size_t flag_bytes = p->ncomp >= 2 ? half_tiles : 0;
+  const size_t list_bytes = p->ncomp == 2 ? (half_tiles + 3) * sizeof(int) : 0;
+  set_layout(c, true);
+  if (!padding_fits(c, nrm_bytes + 2 * flag_bytes + list_bytes)) set_layout(c, false);
   const size_t fb = c->len * c->es;
   if ((rc = dev_alloc(c, (void **)&c->buf[0], fb)) || (rc = dev_alloc(c, (void **)&c->buf[1], fb)) ||
-      (p->ncomp >= 2 && (rc = dev_alloc(c, (void **)&c->nrm, 4 * c->fs * sizeof(float)))) ||
-      (p->ncomp >= 2 &&
-       (rc = dev_alloc(c, (void **)&c->flags, 2 * (size_t)k.tiles_x * k.tiles_y * p->nz))) ||
-      (p->ncomp == 2 &&
-       (rc = dev_alloc(c, (void **)&c->ilist, (2 * (size_t)k.tiles_x * k.tiles_y * p->nz + 3) * sizeof(int)))) ||
-      (p->ncomp == 2 &&
-       (rc = dev_alloc(c, (void **)&c->flags_alt, 2 * (size_t)k.tiles_x * k.tiles_y * p->nz))) ||
+      (nrm_bytes && (rc = dev_alloc(c, (void **)&c->nrm, nrm_bytes))) ||
+      (flag_bytes && (rc = dev_alloc(c, (void **)&c->flags, flag_bytes))) ||
+      (list_bytes && (rc = dev_alloc(c, (void **)&c->ilist, list_bytes))) ||
+      (p->ncomp == 2 && (rc = dev_alloc(c, (void **)&c->flags_alt, flag_bytes))) ||
       (p->storage == TSLB_STORAGE_FX16 && (rc = dev_alloc(c, (void **)&c->sat, 256))) ||
       (rc = dev_alloc(c, (void **)&c->part, (size_t)kRedBlocks * NRED * sizeof(double))) ||
       (rc = dev_alloc(c, (void **)&c->red, NRED * sizeof(double)))) {
@@ -3292,6 +3308,7 @@ int tslb_create(tslb_ctx **out, const tslb_params *p) {
     return fail(rc, msg);
   }
   // zero state: rho-1 = 0, all moments 0
+  (void)hipGetLastError();
   for (int b = 0; b < 2; b++)
     fill(c->stream, c->buf[b], 0.f, (long long)(fb / 4));
   if (c->sat) fill(c->stream, c->sat, 0.f, 1);

@@ -1,8 +1,9 @@
 // tslb.hip -- MI355X (gfx950) TSLB library: HIP kernels and the C ABI of
 // include/tslb.h.
 //
-// State: SoA moment fields on the device, Fortran (i fastest) order, two
-// buffers (source / destination of a step).  Field 0 holds rho-1 (shifted
+// State: moments on the device, ten of them interleaved in rows of 64 nodes, phi
+// a plain field (Fortran order, i fastest); host arrays and files hold plain
+// fields.  Two buffers (source / destination of a step).  Field 0 holds rho-1 (shifted
 // density), so that the FP32 sums of the fused kernel keep their precision;
 // the host interface converts to rho.
 //
@@ -302,7 +303,7 @@ __device__ __forceinline__ float dec(S x, const Params &p, int g) {
 // 32 KiB (found by timing: copying 20 KiB records in random order moves 5.1
 // TB/s when a record is contiguous and 6.1 TB/s when its eight rows lie 32 KiB
 // apart; 16 and 64 KiB are close, 8 and 128 KiB lose it).  So the eight rows of
-// a 64x8 tile-plane sit 32 KiB apart (`kPitch`) and a block opens its own pages
+// a 64x8 tile-plane sit 32 KiB apart (`kLineBytes`) and a block opens its own pages
 // only; 12 tiles (25 in 16-bit storage) share the eight 32 KiB lines of such a
 // superpage.  The access pattern of the fused pass alone (loads with halo, nt
 // stores, no arithmetic) takes, plain fields / rows in sequence / superpages:
@@ -2200,7 +2201,7 @@ __global__ __launch_bounds__(NTHR) void k_iface_list(const S *__restrict__ phi, 
 // takes a block 13 us, most of it latency; while the list leaves blocks of the
 // grid idle, a run's planes go to several (24^3: 13.4 -> 6 us a step).  The plane
 // loop is unrolled over the longest run (ring slots at constant offsets) and
-// held to 80 VGPRs, which keeps three blocks per CU (51 KiB of LDS each).
+// held to 80 VGPRs, which keeps six blocks per CU (26 KiB of LDS each).
 template <typename S>
 __global__ __launch_bounds__(HNT) __attribute__((amdgpu_waves_per_eu(6, 8))) void k_curv_list(const S *__restrict__ phi, float *__restrict__ kap,
                                                     uint8_t *__restrict__ flags, const int *__restrict__ cnt,
@@ -3121,9 +3122,10 @@ void set_layout(tslb_ctx *c, bool padded) {
 // for a mask (8 bytes a node while it is set) or for a closure (48 more) that plain
 // fields leave room for; 256 MiB of slack cover the allocations' own rounding.
 bool padding_fits(const tslb_ctx *c, size_t fixed) {
+  const size_t padded = 2 * c->len * c->es + fixed, plain = 2 * (NIL + 1) * c->fs * c->es + fixed;
+  if (padded < plain + (64u << 20)) return true;  // not worth the query (12 us of the 90 that creating 24^3 takes)
   size_t avail = 0, total = 0;
   if (hipMemGetInfo(&avail, &total) != hipSuccess) return (void)hipGetLastError(), true;
-  const size_t padded = 2 * c->len * c->es + fixed, plain = 2 * (NIL + 1) * c->fs * c->es + fixed;
   for (const size_t later : {0 * c->n, 8 * c->n, 56 * c->n})
     if (plain + later <= avail && padded + later + (256u << 20) > avail) return false;
   return true;

@@ -3,7 +3,7 @@
  *
  * The thread-safe recursive-regularized D3Q27 lattice Boltzmann step (TSLB) for
  * one- and two-component flow on one GPU.  The state lives on the device as
- * structure-of-arrays moment fields (rho, u, v, w, Pi^neq (6), phi); one step is
+ * moment fields (rho, u, v, w, Pi^neq (6), phi); one step is
  * a fused moment-space collide + pull-stream.  Host arrays are Fortran-ordered
  * (1:nx,1:ny,1:nz), i fastest, and stay owned by the caller; nothing is
  * retained after a call returns.

@@ -61,7 +61,7 @@ int grad_rows(tslb_closure *m, int64_t nb) {
   return (int)(groups < m->ncu ? groups : m->ncu);
 }
 
-// largest batch whose columns are kept for k_mlp_wgrad: four slices (see there)
+// largest batch whose columns are kept for k_mlp_wgrad: eight slices (see there)
 constexpr int64_t kColsMax = kWgradWaves * kSlice;
 
 int ensure_train(tslb_closure *m, int64_t nb, bool indices) {

@@ -272,7 +272,7 @@ __global__ __launch_bounds__(256, 4) void k_mlp_infer(const float *__restrict__ 
 // groups.  inv = 1/(t_scale^2 * batch).
 //
 // Latency bounds it: a batch of 16384 is one group per CU (256 groups), and
-// takes 18 us, k_mlp_update 4.5 us.  One wave per tile, 13.6 MB of BF16
+// takes 17 us, k_mlp_update 5 us.  One wave per tile, 13.6 MB of BF16
 // activations written for a second kernel that added dW with atomics, took 29 +
 // 15.5 us, and the indices, two fills, Adam and the packing a launch each, 15 us
 // more.  The weights are in LDS as they do not fit the registers: spilled, they
@@ -617,13 +617,16 @@ __global__ __launch_bounds__(1024) void k_mlp_update(const float *__restrict__ p
 // The rounding of these sums decides what comes out of a training: one other
 // bit of a gradient is 1e-5 in the weights and 3e-3 in the outputs 100 steps
 // on.  Slices of 512 added with atomics gave the same sums, bit for bit with
-// one or two slices and in most runs with three or four (a partial one arrived
-// first); from five on no two runs agreed, and k_mlp_update's sums, in groups of
-// 64, lie as close to each as they to one another.  So the line is four slices.
-// Latency bounds it: one read of the columns, all of a slice in flight, 16
-// dependent MFMAs and Adam.  A step of 1024 samples takes 16.7 us, of 2048 19.0 us
-// (k_mlp_update's way 14.7 and 15.1; 31 and 32 us with atomics).
-constexpr int kSlice = 512, kWgradJobs = 4 + 20 + 20 + 5, kWgradWaves = 4;
+// one or two slices and in many runs with up to five (a partial one arrived
+// first: 2088 samples, 22 steps: outputs 7e-9 from a run of theirs, theirs 1e-8
+// from one another, k_mlp_update's 7e-7, in the median).  From nine on
+// k_mlp_update's sums, in groups of 64, lie as close to a run of theirs as two of
+// theirs to one another (4227 samples, 41 steps: 2e-5, theirs 3e-4).  So the line
+// is eight slices.  Latency bounds it: one read of the columns, all of a slice in
+// flight, 16 dependent MFMAs and Adam.  A step of 1024 samples takes 16.7 us, of
+// 2048 19.1, of 4096 23.7 (k_mlp_update's way 14.7, 15.1 and 16.2; with atomics
+// 31, 32 and 35).
+constexpr int kSlice = 512, kWgradJobs = 4 + 20 + 20 + 5, kWgradWaves = 8;
 struct WgradJob {
   int layer;  // 1..4
   int mb;     // output-feature block (rows of delta)

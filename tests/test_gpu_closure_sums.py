@@ -35,7 +35,7 @@ def test_trained_weights_bit_for_bit(nb):
     assert np.array_equal(got, want), np.abs(got - want).max()
 
 
-@pytest.mark.parametrize("nb", [1024, 1536, 2048])
+@pytest.mark.parametrize("nb", [1024, 1536, 2048, 4096])
 def test_gradient_is_the_sum_of_its_slices(nb):
     """Slices of 512, each a gradient of its own, added in order.  The weight of a
     sample is 1/nb, a power of two apart for the scaled batches below, so the

@@ -2561,9 +2561,14 @@ __global__ __launch_bounds__(256) void k_jet_bc(const S *__restrict__ src, S *__
     const float r = 1.f + sm[0];
     const float inv = 1.f / r;
     const float u = sm[1] * inv, v = sm[2] * inv, w = sm[3] * inv;
-    const float tt = sm[0] * (1.f / 3.f);
-    const float out[10] = {sm[0], u, v, w, sm[4] - tt - r * u * u, sm[5] - tt - r * v * v,
-                           sm[6] - tt - r * w * w, sm[7] - r * u * v, sm[8] - r * u * w, sm[9] - r * v * w};
+    // less (rho-1)/3, fused but for Pyy and Pzz in FX16: which, the compiler chose
+    // by the code around it, so it is written out, as each storage type has had it
+    auto trace = [&](int q) {
+      if (std::is_same<S, fx16_t>::value && q > 4) return sum_of_rounded(sm[q], sm[0] * (-1.f / 3.f));
+      return fmaf(sm[0], -1.f / 3.f, sm[q]);
+    };
+    const float out[10] = {sm[0], u, v, w, trace(4) - r * u * u, trace(5) - r * v * v,
+                           trace(6) - r * w * w, sm[7] - r * u * v, sm[8] - r * u * w, sm[9] - r * v * w};
 #pragma unroll
     for (int q = 0; q < 10; q++) stf(dst, q, i, j, zy, out[q], p);
   }

@@ -844,9 +844,11 @@ struct FeatPacked {
 // A 64x4 block marches a z-chunk.  It keeps four planes of its 66x6 footprint
 // in an LDS ring (25 KiB; the plane two ahead loads into registers meanwhile)
 // and forms the 12 sums of a node from 104 LDS reads, in the order of the
-// directions.  One thread per node reading its 26 neighbours from memory
-// took 79 us at 128^3 for its addresses and L1 reads; this one takes 34 us (84 MB
-// written and 34 MB read: 24 us at the rate of a copy).
+// directions, those with a zero coefficient too: a NaN or an infinity of any
+// neighbour shows in all components (2 us of the 33).  One thread per node
+// reading its 26 neighbours from memory took 79 us at 128^3 for its addresses
+// and L1 reads; this one takes 33 us (84 MB written and 34 MB read: 24 us at the
+// rate of a copy).
 constexpr int FTX = 64, FTY = 4, FSW = FTX + 2, FSH = FTY + 2, FNSLOT = FSW * FSH, FNT = FTX * FTY;
 static_assert(FNSLOT <= 2 * FNT, "at most two footprint slots per thread");
 template <typename Src, bool PHI, typename Out>
@@ -906,9 +908,9 @@ __global__ __launch_bounds__(FNT) void k_features(Src f, Params p, int fu, int f
 #pragma unroll
       for (int q = 0; q < NQ; q++) {
         const float v = s[q * FNSLOT];
-        if (kCX[l]) g[q][0] = fmaf(w3 * (float)kCX[l], v, g[q][0]);
-        if (kCY[l]) g[q][1] = fmaf(w3 * (float)kCY[l], v, g[q][1]);
-        if (kCZ[l]) g[q][2] = fmaf(w3 * (float)kCZ[l], v, g[q][2]);
+        g[q][0] = fmaf(w3 * (float)kCX[l], v, g[q][0]);
+        g[q][1] = fmaf(w3 * (float)kCY[l], v, g[q][1]);
+        g[q][2] = fmaf(w3 * (float)kCZ[l], v, g[q][2]);
       }
     }
     const float v[kMlpNF] = {g[0][0],
